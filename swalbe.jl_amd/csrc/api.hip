@@ -177,25 +177,27 @@ int ensure_kappa(swalbe_state* st, int n, int m, double hmin) {
   return SWALBE_OK;
 }
 
-// host <-> device copies of a field in the state's element type; the
-// distribution planes sit fstride elements apart on the device.
-int copy_h2d(swalbe_state* st, int field, void* dst, const void* src) {
-  const Film& F = st->film;
-  hipError_t e;
-  if (is_dist(field))
-    e = hipMemcpy2D(dst, F.fstride * F.esz, src, F.N * F.esz, F.N * F.esz, kQ, hipMemcpyHostToDevice);
-  else
-    e = hipMemcpy(dst, src, F.N * F.esz, hipMemcpyHostToDevice);
-  return e == hipSuccess ? SWALBE_OK : hip_fail(e, "copy to device");
+// Encoding offsets of a field's planes (all 0 for FP64 and plain fields).
+void plane_offsets(const Film& F, int field, double off[kQ]) {
+  for (int k = 0; k < kQ; ++k) off[k] = enc_offset(F, field, is_dist(field) ? k : 0);
 }
-int copy_d2h(swalbe_state* st, int field, void* dst, const void* src) {
+
+// host <-> device copies of a field: host elements of hes bytes, decoded
+// (`plain`) or as stored; the distribution planes sit fstride elements apart
+// on the device.
+int copy_h2d(swalbe_state* st, int field, void* dst, const void* src, size_t hes, bool plain) {
   const Film& F = st->film;
-  hipError_t e;
-  if (is_dist(field))
-    e = hipMemcpy2D(dst, F.N * F.esz, src, F.fstride * F.esz, F.N * F.esz, kQ, hipMemcpyDeviceToHost);
-  else
-    e = hipMemcpy(dst, src, F.N * F.esz, hipMemcpyDeviceToHost);
-  return e == hipSuccess ? SWALBE_OK : hip_fail(e, "copy to host");
+  double off[kQ];
+  plane_offsets(F, field, off);
+  return field_from_host(dst, F.esz, src, hes, F.N, is_dist(field) ? kQ : 1, F.fstride,
+                         plain ? off : nullptr, st->device, st->stream);
+}
+int copy_d2h(swalbe_state* st, int field, void* dst, const void* src, size_t hes, bool plain) {
+  const Film& F = st->film;
+  double off[kQ];
+  plane_offsets(F, field, off);
+  return field_to_host(dst, hes, src, F.esz, F.N, is_dist(field) ? kQ : 1, F.fstride,
+                       plain ? off : nullptr, st->device, st->stream);
 }
 
 int set_device(swalbe_state* st) {
@@ -232,6 +234,7 @@ int swalbe_create(int32_t Lx, int32_t Ly, int32_t dtype, int32_t kind, swalbe_st
     return SWALBE_EINVAL;
   }
   swalbe_state* st = new swalbe_state();
+  xfer_retain();
   Film& F = st->film;
   F.Lx = Lx;
   F.Ly = Ly;
@@ -311,6 +314,7 @@ int swalbe_destroy(swalbe_state* st) {
     if (p) hipFree(p);
   if (st->own_stream) hipStreamDestroy(st->own_stream);
   delete st;
+  xfer_release();
   return SWALBE_OK;
 }
 
@@ -345,15 +349,7 @@ int swalbe_upload(swalbe_state* st, int32_t field, const void* host, size_t byte
   if (field == SWALBE_FOUT || field == SWALBE_FTEMP) unalias_for_write(F, field);
   int64_t c2;
   void* dst = field_ptr(st, field, &c2);
-  std::vector<unsigned char> tmp((size_t)count * F.esz);
-  for (int64_t i = 0; i < count; ++i) {
-    const double v = hes == 8 ? ((const double*)host)[i] : (double)((const float*)host)[i];
-    const double off = enc_offset(F, field, (int)(i / F.N));
-    if (F.esz == 8) ((double*)tmp.data())[i] = v - off;
-    else ((float*)tmp.data())[i] = (float)(v - off);
-  }
-  SW_HIP(hipStreamSynchronize(st->stream));
-  return copy_h2d(st, field, dst, tmp.data());
+  return copy_h2d(st, field, dst, host, hes, true);
 }
 
 // Stored representation of a field (esz bytes per element; FP32 heights and
@@ -376,8 +372,7 @@ int swalbe_download_raw(swalbe_state* st, int32_t field, void* host, size_t byte
     set_error("swalbe_download_raw: byte count must be the stored size (elements x 4 or 8)");
     return SWALBE_EINVAL;
   }
-  SW_HIP(hipStreamSynchronize(st->stream));
-  return copy_d2h(st, field, host, src);
+  return copy_d2h(st, field, host, src, F.esz, false);
 }
 
 int swalbe_upload_raw(swalbe_state* st, int32_t field, const void* host, size_t bytes) {
@@ -399,8 +394,7 @@ int swalbe_upload_raw(swalbe_state* st, int32_t field, const void* host, size_t 
   if (field == SWALBE_FOUT || field == SWALBE_FTEMP) unalias_for_write(F, field);
   int64_t c2;
   void* dst = field_ptr(st, field, &c2);
-  SW_HIP(hipStreamSynchronize(st->stream));
-  return copy_h2d(st, field, dst, host);
+  return copy_h2d(st, field, dst, host, F.esz, false);
 }
 
 // FP32 reference height and gravity of the deviation storage (href = 0 for FP64).
@@ -454,17 +448,7 @@ int swalbe_download(swalbe_state* st, int32_t field, void* host, size_t bytes) {
     set_error("swalbe_download: byte count does not match the field size");
     return SWALBE_EINVAL;
   }
-  std::vector<unsigned char> tmp((size_t)count * F.esz);
-  SW_HIP(hipStreamSynchronize(st->stream));
-  if (int rc = copy_d2h(st, field, tmp.data(), src)) return rc;
-  for (int64_t i = 0; i < count; ++i) {
-    const double raw = F.esz == 8 ? ((double*)tmp.data())[i] : (double)((float*)tmp.data())[i];
-    const double off = enc_offset(F, field, (int)(i / F.N));
-    const double v = off == 0.0 ? raw : raw + off;
-    if (hes == 8) ((double*)host)[i] = v;
-    else ((float*)host)[i] = (float)v;
-  }
-  return SWALBE_OK;
+  return copy_d2h(st, field, host, src, hes, true);
 }
 
 int swalbe_fill(swalbe_state* st, int32_t field, double value) {
@@ -498,30 +482,23 @@ int swalbe_set_reference_height(swalbe_state* st, double href, double g) {
     set_error("swalbe_set_reference_height: non-finite value");
     return SWALBE_EINVAL;
   }
-  // re-encode resident height and distributions through the host (rare call)
+  if (int rc = set_device(st)) return rc;
+  // re-encode the resident height and distributions in place
   const int ids[] = {SWALBE_HEIGHT, SWALBE_FOUT, SWALBE_FTEMP, SWALBE_FEQ};
-  std::vector<std::vector<double>> keep;
   const bool aliased = F.fout_buf == F.ftemp_buf;
-  for (int id : ids) {
-    const int64_t count = is_dist(id) ? 9 * F.N : F.N;
-    keep.emplace_back(count);
-    if (id == SWALBE_FTEMP && aliased) continue;
-    if (int rc = swalbe_download(st, id, keep.back().data(), count * 8)) return rc;
-  }
+  double from[4][kQ], to[4][kQ];
+  for (int i = 0; i < 4; ++i) plane_offsets(F, ids[i], from[i]);
   F.href = href;
   F.g_enc = g;
   F.enc = make_enc(href, g);
-  for (size_t i = 0; i < 4; ++i) {
-    const int id = ids[i];
-    if (id == SWALBE_FTEMP && aliased) continue;
-    // write without un-aliasing: re-encoding keeps buffer identities
+  for (int i = 0; i < 4; ++i) {
+    if (ids[i] == SWALBE_FTEMP && aliased) continue;
+    plane_offsets(F, ids[i], to[i]);
     int64_t count;
-    void* dst = field_ptr(st, id, &count);
-    std::vector<unsigned char> tmp((size_t)count * 4);
-    for (int64_t j = 0; j < count; ++j)
-      ((float*)tmp.data())[j] = (float)(keep[i][j] - enc_offset(F, id, (int)(j / F.N)));
-    if (int rc = copy_h2d(st, id, dst, tmp.data())) return rc;
+    float* p = (float*)field_ptr(st, ids[i], &count);
+    launch_reencode(p, F.N, is_dist(ids[i]) ? kQ : 1, F.fstride, from[i], to[i], st->stream);
   }
+  SW_HIP(hipGetLastError());
   return SWALBE_OK;
 }
 

@@ -300,6 +300,7 @@ void release(swalbe_batch* b) {
   if (b->dl_stream) hipStreamDestroy(b->dl_stream);
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
+  xfer_release();
 }
 
 // ---------------------------------------------------------------- autotuner
@@ -431,6 +432,7 @@ int swalbe_batch_create(int32_t dtype, size_t capacity_bytes, int32_t max_films,
   if (!out || dtype != SWALBE_F32 || capacity_bytes < kAlign || max_films < 1)
     return bad("swalbe_batch_create: FP32 only, capacity and max_films must be positive");
   swalbe_batch* b = new swalbe_batch();
+  xfer_retain();
   hipGetDevice(&b->device);
   hipError_t e = hipMalloc(&b->arena, capacity_bytes);
   if (e != hipSuccess) {
@@ -717,7 +719,6 @@ int swalbe_batch_download(swalbe_batch* b, int32_t slot, int32_t field, void* ho
   if (bytes == (size_t)count * 8) hes = 8;
   else if (bytes == (size_t)count * 4) hes = 4;
   else return bad("swalbe_batch_download: byte count does not match the field size");
-  std::vector<float> tmp(count);
   // a finished film is not touched by later launches: wait only for the
   // enqueue call that ran its last step, so the copy overlaps newer steps
   if (n > 0 && b->counter >= d.end) {
@@ -725,19 +726,10 @@ int swalbe_batch_download(swalbe_batch* b, int32_t slot, int32_t field, void* ho
   } else {
     SW_HIP(hipStreamSynchronize(b->stream));
   }
-  if (field == SWALBE_FOUT)
-    SW_HIP(hipMemcpy2DAsync(tmp.data(), N * 4, src, d.fstride * 4, N * 4, 9,
-                            hipMemcpyDeviceToHost, b->dl_stream));
-  else
-    SW_HIP(hipMemcpyAsync(tmp.data(), src, N * 4, hipMemcpyDeviceToHost, b->dl_stream));
-  SW_HIP(hipStreamSynchronize(b->dl_stream));
-  for (int64_t i = 0; i < count; ++i) {
-    const double o = field == SWALBE_FOUT ? (double)s.enc.R[i / N] : off;
-    const double v = (double)tmp[i] + o;
-    if (hes == 8) ((double*)host)[i] = v;
-    else ((float*)host)[i] = (float)v;
-  }
-  return SWALBE_OK;
+  const int planes = field == SWALBE_FOUT ? kQ : 1;
+  double offs[kQ];
+  for (int k = 0; k < kQ; ++k) offs[k] = field == SWALBE_FOUT ? (double)s.enc.R[k] : off;
+  return field_to_host(host, hes, src, 4, N, planes, d.fstride, offs, b->device, b->dl_stream);
 }
 
 int swalbe_batch_stats(swalbe_batch* b, int32_t* nfilms, int64_t* nodes, size_t* bytes_used,

@@ -970,6 +970,7 @@ int swalbe1d_create(int32_t L, int32_t dtype, int32_t kind, swalbe_film1d** out)
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "swalbe1d_create: hipGetDevice");
   swalbe_film1d* s = new swalbe_film1d();
+  swalbe::xfer_retain();
   s->L = L;
   s->dtype = dtype;
   s->kind = kind;
@@ -1032,6 +1033,7 @@ int swalbe1d_destroy(swalbe_film1d* s) {
       if (e == hipSuccess) e = ef;
     }
   delete s;
+  swalbe::xfer_release();
   if (e != hipSuccess) return hip_fail(e, "swalbe1d_destroy");
   return SWALBE_OK;
 }
@@ -1059,15 +1061,8 @@ int swalbe1d_upload(swalbe_film1d* s, int32_t field, const void* host, size_t by
       if (int rc = alloc1(s, o, s->L)) return rc;
   }
   split_dists(s, field);
-  std::vector<unsigned char> tmp((size_t)n * s->esz);
-  for (int64_t i = 0; i < n; ++i) {
-    const double v = hes == 8 ? ((const double*)host)[i] : (double)((const float*)host)[i];
-    if (s->esz == 8) ((double*)tmp.data())[i] = v;
-    else ((float*)tmp.data())[i] = (float)v;
-  }
-  SW_HIP1(hipStreamSynchronize(s->stream));
-  SW_HIP1(hipMemcpy(field1(s, field), tmp.data(), tmp.size(), hipMemcpyHostToDevice));
-  return SWALBE_OK;
+  return swalbe::field_from_host(field1(s, field), s->esz, host, hes, n, 1, n, nullptr, s->device,
+                                 s->stream);
 }
 
 int swalbe1d_download(swalbe_film1d* s, int32_t field, void* host, size_t bytes) {
@@ -1079,15 +1074,7 @@ int swalbe1d_download(swalbe_film1d* s, int32_t field, void* host, size_t bytes)
   const int64_t n = is_dist1(field) ? 3 * (int64_t)s->L : s->L;
   const size_t hes = bytes == (size_t)n * 8 ? 8 : (bytes == (size_t)n * 4 ? 4 : 0);
   if (!hes) return bad1("swalbe1d_download: byte count does not match the field size");
-  std::vector<unsigned char> tmp((size_t)n * s->esz);
-  SW_HIP1(hipStreamSynchronize(s->stream));
-  SW_HIP1(hipMemcpy(tmp.data(), src, tmp.size(), hipMemcpyDeviceToHost));
-  for (int64_t i = 0; i < n; ++i) {
-    const double v = s->esz == 8 ? ((double*)tmp.data())[i] : (double)((float*)tmp.data())[i];
-    if (hes == 8) ((double*)host)[i] = v;
-    else ((float*)host)[i] = (float)v;
-  }
-  return SWALBE_OK;
+  return swalbe::field_to_host(host, hes, src, s->esz, n, 1, n, nullptr, s->device, s->stream);
 }
 
 int swalbe1d_fill(swalbe_film1d* s, int32_t field, double value) {

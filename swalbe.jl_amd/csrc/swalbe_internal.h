@@ -222,6 +222,24 @@ void launch_measure(const T* h, double href, int Lx, int Ly, double thresh, int 
                     double cos_s, const T* theta, uint8_t* mask, double* partials, int nparts,
                     double* out, hipStream_t s);
 
+// ---------------------------------------------------------------- host transfers
+// A field of `planes` planes of n elements (plane k at dev + k * stride
+// elements; `off`: one encoding offset per plane, or null) to and from a
+// contiguous host array whose elements are hes bytes (8: double, 4: float);
+// des is the device element size.  Equal element types without an offset are
+// copied bit for bit.  Ordered after earlier work on `s`; complete on return.
+int field_to_host(void* host, size_t hes, const void* dev, size_t des, int64_t n, int planes,
+                  int64_t stride, const double* off, int device, hipStream_t s);
+int field_from_host(void* dev, size_t des, const void* host, size_t hes, int64_t n, int planes,
+                    int64_t stride, const double* off, int device, hipStream_t s);
+// FP32 planes re-encoded in place from one set of offsets to another.
+void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const double* from,
+                     const double* to, hipStream_t s);
+// Called once per film or batch at creation and destruction: the pinned
+// transfer buffers are kept while any exists.
+void xfer_retain();
+void xfer_release();
+
 // ---------------------------------------------------------------- errors
 void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
