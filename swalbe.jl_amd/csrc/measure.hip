@@ -133,18 +133,24 @@ __global__ __launch_bounds__(kMT) void k_measure(const T* __restrict__ h, double
   }
 }
 
+// One wave folds the blocks' partials in a fixed order (lane l takes l,
+// l + 64, ..., then a tree).
 // out = {count, max, area, reduced energy}; the energy subtracts
 // count · cos πθ (scalar θ) or Σ cos πθ over the wet nodes (θ field)
 __global__ void k_measure_finish(const double* __restrict__ partials, int nparts, double cos_s,
                                  int theta_field, double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
   double c = 0.0, m = -__builtin_inf(), s = 0.0, k = 0.0;
-  for (int b = 0; b < nparts; ++b) {
+  for (int b = threadIdx.x; b < nparts; b += 64) {
     c += partials[4 * b + 0];
     m = partials[4 * b + 1] > m ? partials[4 * b + 1] : m;
     s += partials[4 * b + 2];
     k += partials[4 * b + 3];
   }
+  c = wsum(c);
+  m = wmax(m);
+  s = wsum(s);
+  k = wsum(k);
+  if (threadIdx.x != 0) return;
   out[0] = c;
   out[1] = m;
   out[2] = s;
