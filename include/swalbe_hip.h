@@ -423,8 +423,10 @@ typedef struct swalbe1d_step_opts {
     int32_t body;            /* inclination!(α, state) after the force sum */
     int32_t bound;           /* bounce-back walls (BORDER1/2); mass Σ(h - interior h) */
     int32_t materialize;     /* afterwards pressure, h∇p, slip, kbt, F, feq hold the last step's */
-    int32_t variant;         /* 0 = resident when the film fits in LDS, else one launch per
-                                step; 1 = one launch per step; 2 = resident (error if too big) */
+    int32_t variant;         /* 0 = several steps per launch in registers (with `threads` set:
+                                resident when the film fits in LDS, else one launch per step);
+                                1 = one launch per step; 2 = resident (error if too big);
+                                every variant gives the same fields */
     uint64_t seed;
     int64_t t0;
     double alpha, body_fac;

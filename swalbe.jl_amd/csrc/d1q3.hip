@@ -3,6 +3,8 @@
 // State_1D and its kinds (src/initialize.jl:276-341, allocator :587-616) on
 // the GPU, one kernel per reference op, and two fused time loops
 // (src/simulate.jl:98-205, run_gamma :518-560):
+//   * k1_wave: several steps per launch in registers, any L; the last step
+//     of a loop in k1_step, which writes every output (single films).
 //   * k1_step: one launch per step, any L; h on a 3-node halo in LDS.
 //   * k1_resident: the whole film in LDS and every step in one launch, one
 //     workgroup per film.  A film of L nodes needs (6 + 6 [τ != 1]) L words
@@ -421,6 +423,229 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step,
 template <typename T>
 __device__ __forceinline__ __attribute__((address_space(1))) T* glb(T* p) {
   return (__attribute__((address_space(1))) T*)p;
+}
+
+// The (n, m) law of the fused steps: power_broad's products in its order
+// (1 a = a is exact, and the m factors are the first m of the n); the two
+// usual pairs need no loop.
+template <typename T>
+__device__ __forceinline__ T disjoin_law(T a, int n, int m) {
+  if (n == 9 && m == 3) {
+    const T a3 = (a * a) * a;
+    const T a6 = ((a3 * a) * a) * a;
+    return (((a6 * a) * a) * a) - a3;
+  }
+  if (n == 3 && m == 2) {
+    const T a2 = a * a;
+    return a2 * a - a2;
+  }
+  return powbroad(a, n) - powbroad(a, m);
+}
+
+// The value of the lane below / above (DPP wave_shr:1 / wave_shl:1; 0 beyond
+// the wave's ends, whose nodes are halo and never written).
+template <int CTRL>
+__device__ __forceinline__ int dpp_shift(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift(float v) {
+  return __builtin_bit_cast(float, dpp_shift<CTRL>(__builtin_bit_cast(int, v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)dpp_shift<CTRL>((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)dpp_shift<CTRL>((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <typename T>
+__device__ __forceinline__ T from_below(T v) {
+  return dpp_shift<0x138>(v);
+}
+template <typename T>
+__device__ __forceinline__ T from_above(T v) {
+  return dpp_shift<0x130>(v);
+}
+
+// `k` steps of one film in one launch, in registers: wave b holds the window
+// of 64 NPT nodes from b W - 3 k, NPT consecutive nodes per lane, and loses
+// three nodes at each end per step (one per stencil), so that after k steps
+// the W = 64 NPT - 6 k nodes from b W are exact.  Neighbours come from the
+// lane itself or the next lane (DPP): no LDS, no barrier, no traffic between
+// the steps.  Only h and u are written (and f when τ ≠ 1, which the next
+// launch reads); the loop's last step runs in k1_step, which writes every
+// output.
+//
+// What bounds it: FP64 issue (about 100 instructions per node and step, three
+// IEEE divisions among them).  One node per lane takes 0.28 us a step however
+// short the film; the 2.2 us of a launch are shared by its k steps.  Measured
+// against the kernels it replaces for single films (us per step): L = 1024
+// 4.6 in one workgroup's LDS -> 0.51, over up to 256 CUs instead of one;
+// L = 3e6 36.4 with one launch and 64 bytes per node and step -> 12.2, with
+// 6 bytes per node and step.
+// EXTRA: any of the κ, γ, ∇γ fields or walls; RFT: τ ≠ 1; TH: noise.
+template <typename T, int NPT, bool RFT, bool TH, bool EXTRA>
+__global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, int W,
+                                              unsigned long long* dh_keys,
+                                              unsigned long long* wet) {
+  const int lane = threadIdx.x, L = S.L;
+  const int64_t x0 = (int64_t)blockIdx.x * W;         // first node written
+  const int64_t xs = x0 - 3 * k + (int64_t)lane * NPT;  // this lane's first node
+  int xw[NPT];  // wrapped node indices
+  const bool inner = x0 - 3 * k >= 0 && x0 - 3 * k + 64 * NPT <= L;
+#pragma unroll
+  for (int j = 0; j < NPT; ++j) {
+    int64_t x = xs + j;
+    if (!inner) {
+      x %= L;
+      x = x < 0 ? x + L : x;
+    }
+    xw[j] = (int)x;
+  }
+  T h[NPT], u[NPT], t0[NPT], t1[NPT], t2[NPT];
+#pragma unroll
+  for (int j = 0; j < NPT; ++j) {
+    h[j] = ((const T*)S.h_in)[xw[j]];
+    u[j] = ((const T*)S.u_in)[xw[j]];
+    if constexpr (RFT) {
+      t0[j] = ((const T*)S.ft)[xw[j]];
+      t1[j] = ((const T*)S.ft)[L + (int64_t)xw[j]];
+      t2[j] = ((const T*)S.ft)[2 * (int64_t)L + xw[j]];
+    }
+  }
+  T kap[NPT], gam[NPT], gg[NPT], b1[NPT], b2[NPT];
+  const bool walls = EXTRA && S.b1 != nullptr;
+#pragma unroll
+  for (int j = 0; j < NPT; ++j) {
+    kap[j] = EXTRA && S.kap ? ((const T*)S.kap)[xw[j]] : (T)S.kap_s;
+    gam[j] = EXTRA && S.gam ? ((const T*)S.gam)[xw[j]] : (T)S.gamma;
+    if constexpr (EXTRA) {
+      gg[j] = S.gg ? ((const T*)S.gg)[xw[j]] : T(0);
+      b1[j] = walls ? ((const T*)S.b1)[xw[j]] : T(0);
+      b2[j] = walls ? ((const T*)S.b2)[xw[j]] : T(0);
+    }
+  }
+  const int n = S.n, m = S.m;
+  const T hmin = (T)S.hmin, hcrit = (T)S.hcrit, g = (T)S.g;
+  const T c6mu = (T)S.c6mu, c6d = (T)S.c6d, c3dd = (T)S.c3dd;
+  const T omeg = (T)S.omeg, itau = (T)S.itau;
+  const int own0 = 3 * k - lane * NPT;  // nodes j with own0 <= j < own0 + W are this wave's
+#pragma unroll 1
+  for (int s = 0; s < k; ++s) {
+    if (dh_keys || wet) {  // series over the step's input height
+      unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
+#pragma unroll
+      for (int j = 0; j < NPT; ++j)
+        if (j >= own0 && j < own0 + W && xs + j < L) {
+          const double hv = (double)h[j];
+          const unsigned long long q = dkey(hv);
+          kmax = q > kmax ? q : kmax;
+          kmin = q < kmin ? q : kmin;
+          cnt += hv > S.wet_thresh ? 1ull : 0ull;
+        }
+      for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
+        kmax = a > kmax ? a : kmax;
+        kmin = b < kmin ? b : kmin;
+        cnt += __shfl_xor(cnt, o);
+      }
+      if (lane == 0) {
+        if (dh_keys) {
+          atomicMax(&dh_keys[2 * s], kmax);
+          atomicMin(&dh_keys[2 * s + 1], kmin);
+        }
+        if (wet && cnt) atomicAdd(&wet[s], cnt);
+      }
+    }
+    T p[NPT];
+    {
+      const T hl = from_below(h[NPT - 1]), hr = from_above(h[0]);
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) {
+        const T hm = j > 0 ? h[j > 0 ? j - 1 : 0] : hl;
+        const T hp = j < NPT - 1 ? h[j < NPT - 1 ? j + 1 : 0] : hr;
+        const T a = hmin / (h[j] + hcrit);
+        const T v = -gam[j] * (kap[j] * disjoin_law(a, n, m));
+        p[j] = v - gam[j] * ((hm - T(2) * h[j]) + hp);
+      }
+    }
+    // forces and the collision at the source: f0 -> h, f1 -> u, f2 apart
+    T f2[NPT];
+    {
+      const T pl = from_below(p[NPT - 1]), pr = from_above(p[0]);
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) {
+        const T pm = j > 0 ? p[j > 0 ? j - 1 : 0] : pl;
+        const T pp = j < NPT - 1 ? p[j < NPT - 1 ? j + 1 : 0] : pr;
+        const T hh = h[j];
+        const T hgp = (hh * T(-0.5)) * (pm - pp);
+        T F = -hgp - slip_node(hh, u[j], c6mu, c6d, c3dd);
+        if constexpr (TH)
+          F = F - noise_node<T>(S.seed, step0 + (uint64_t)s, xw[j]) *
+                      noise_amp(hh, (T)S.kb26, (T)S.delta);
+        if constexpr (EXTRA) {
+          if (S.gg) F = S.gg_sign < 0 ? F - gg[j] : F + gg[j];
+        }
+        if (S.body) F = F + (hh * (T)S.alpha) * (T)S.fac;
+        T e0, e1, e2;
+        feq_node(hh, u[j], g, e0, e1, e2);
+        if constexpr (RFT) {
+          h[j] = omeg * t0[j] + itau * e0;
+          u[j] = (omeg * t1[j] + itau * e1) + T(0.5) * F;
+          f2[j] = (omeg * t2[j] + itau * e2) - T(0.5) * F;
+        } else {  // τ = 1: 1/τ = 1 and no f_t
+          h[j] = e0;
+          u[j] = e1 + T(0.5) * F;
+          f2[j] = e2 - T(0.5) * F;
+        }
+      }
+    }
+    // pull-stream (bounce-back at walls) and moments
+    {
+      const T fl = from_below(u[NPT - 1]), fr = from_above(f2[0]);
+      T bl = T(0), br = T(0);
+      if constexpr (EXTRA) {
+        bl = from_below(b1[NPT - 1]);
+        br = from_above(b2[0]);
+      }
+      T prev1 = fl, prevb = bl;  // f1 and b1 of the node before
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) {
+        const T s1 = u[j], s2 = f2[j];
+        const T f0 = h[j];
+        T f1 = prev1, fb = j < NPT - 1 ? f2[j < NPT - 1 ? j + 1 : 0] : fr;
+        if constexpr (EXTRA) {
+          if (walls) {
+            const T bp = j < NPT - 1 ? b2[j < NPT - 1 ? j + 1 : 0] : br;
+            f1 = (f1 - f1 * prevb) + s2 * b2[j];
+            fb = (fb - fb * bp) + s1 * b1[j];
+          }
+          prevb = b1[j];
+        }
+        prev1 = s1;
+        if constexpr (RFT) {
+          t0[j] = f0;
+          t1[j] = f1;
+          t2[j] = fb;
+        }
+        const T hn = (f0 + f1) + fb;
+        h[j] = hn;
+        u[j] = (f1 - fb) / hn;
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NPT; ++j)
+    if (j >= own0 && j < own0 + W && xs + j < L) {
+      ((T*)S.h_out)[xw[j]] = h[j];
+      ((T*)S.u_out)[xw[j]] = u[j];
+      if constexpr (RFT) {
+        ((T*)S.f_out)[xw[j]] = t0[j];
+        ((T*)S.f_out)[L + (int64_t)xw[j]] = t1[j];
+        ((T*)S.f_out)[2 * (int64_t)L + xw[j]] = t2[j];
+      }
+    }
 }
 
 // Whole films in LDS: workgroup b steps film table[b] through nsteps steps.
@@ -1384,10 +1609,82 @@ hipError_t launch_resident(const Film1* d_table, int nfilms, int64_t nsteps, int
   return launch_resident_t<T, 1024>(d_table, nfilms, nsteps, lds, st);
 }
 
-// one launch per step (any L): the moments and distributions ping-pong
-// between the two buffers of each
+// Nodes per lane and steps per launch of k1_wave for a film of L nodes: the
+// pair with the smallest modelled time per step.  A launch costs 1.2 us and
+// 0.5 us per node of a lane (its strided loads and stores), 0.8 us more where
+// a SIMD takes more than one wave; a step 0.28 us per node of a lane while a
+// SIMD holds one wave (0.24 and 0.22 us with 4 and 8 nodes, whose chains
+// overlap), 0.22 us per node and wave where it holds more.  Fitted to FP64
+// films of 64 to 3e6 nodes over npt 1-8 and k 4-24; the choice is within 7 %
+// of the best pair measured at each (at 1024 nodes (1, 10): 0.51 us a step
+// against 0.64 for (2, 18); at 2e5 (4, 8): 1.50 against 1.69 for (2, 8); at
+// 3e6 (8, 8): 12.2 against 12.5 for (4, 8)).
+struct WaveShape {
+  int npt, k;
+};
+WaveShape wave_shape(int L, int most, int simds) {
+  WaveShape best{1, 1};
+  double least = 1e30;
+  for (int npt = 1; npt <= most; npt *= 2)
+    for (int k = 2; k <= 32; k += 2) {
+      const int W = 64 * npt - 6 * k;
+      if (W < 4) break;
+      const int per = (int)(((int64_t)(L - 1) / W + simds) / simds);  // waves per SIMD
+      const double alone = npt <= 2 ? 0.28 : npt == 4 ? 0.24 : 0.22;
+      const double node = per == 1 ? alone : std::max(alone, 0.22 * per);
+      const double t = (1.2 + 0.5 * npt + (per > 1 ? 0.8 : 0.0)) / k + npt * node;
+      if (t < least) {
+        least = t;
+        best = WaveShape{npt, k};
+      }
+    }
+  return best;
+}
+
+template <typename T, int NPT, bool RFT, bool TH, bool EXTRA>
+void launch_wave_t(const Film1& S, uint64_t step, int k, unsigned long long* kk,
+                   unsigned long long* ww, hipStream_t st) {
+  const int W = 64 * NPT - 6 * k;
+  hipLaunchKernelGGL((k1_wave<T, NPT, RFT, TH, EXTRA>), dim3((S.L - 1) / W + 1), dim3(64), 0, st,
+                     S, step, k, W, kk, ww);
+}
+
+template <typename T, int NPT>
+void launch_wave_n(const Film1& S, uint64_t step, int k, unsigned long long* kk,
+                   unsigned long long* ww, hipStream_t st) {
+  const bool extra = S.kap || S.gam || S.gg || S.b1;
+  if (S.read_ft) {
+    if (S.thermal)
+      extra ? launch_wave_t<T, NPT, true, true, true>(S, step, k, kk, ww, st)
+            : launch_wave_t<T, NPT, true, true, false>(S, step, k, kk, ww, st);
+    else
+      extra ? launch_wave_t<T, NPT, true, false, true>(S, step, k, kk, ww, st)
+            : launch_wave_t<T, NPT, true, false, false>(S, step, k, kk, ww, st);
+  } else if (S.thermal) {
+    extra ? launch_wave_t<T, NPT, false, true, true>(S, step, k, kk, ww, st)
+          : launch_wave_t<T, NPT, false, true, false>(S, step, k, kk, ww, st);
+  } else {
+    extra ? launch_wave_t<T, NPT, false, false, true>(S, step, k, kk, ww, st)
+          : launch_wave_t<T, NPT, false, false, false>(S, step, k, kk, ww, st);
+  }
+}
+
+// k steps of k1_wave; kk, ww: the series slots of its first step
+template <typename T>
+void launch_wave(const Film1& S, uint64_t step, int npt, int k, unsigned long long* kk,
+                 unsigned long long* ww, hipStream_t st) {
+  if (npt == 8) launch_wave_t<T, 8, false, false, false>(S, step, k, kk, ww, st);
+  else if (npt == 4) launch_wave_n<T, 4>(S, step, k, kk, ww, st);
+  else if (npt == 2) launch_wave_n<T, 2>(S, step, k, kk, ww, st);
+  else launch_wave_n<T, 1>(S, step, k, kk, ww, st);
+}
+
+// The loop in launches of k1_step (any L) or, with `wave`, of k1_wave for
+// every step but the last (and but the steps that a mass record or snapshot
+// falls between); the moments and distributions ping-pong between the two
+// buffers of each
 int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
-                  const swalbe1d_step_opts* o) {
+                  const swalbe1d_step_opts* o, bool wave) {
   unsigned long long *keys = nullptr, *wet = nullptr;
   double* mass = nullptr;
   void* snap = nullptr;
@@ -1409,8 +1706,22 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
     // nodes (threads) per workgroup of k1_step: opts.threads, else 256
     const int nbt = o->threads ? o->threads : 256;
     const int nb = (s->L + nbt * k1_npt(nbt) - 1) / (nbt * k1_npt(nbt));
-    for (int64_t it = 1; it <= nsteps; ++it) {
+    const bool plain = !S.read_ft && !S.thermal && !S.kap && !S.gam && !S.gg && !S.b1;
+    const WaveShape shape = wave_shape(s->L, plain ? 8 : 4, 4 * swalbe::device_cus());
+    // steps from `it` (1-based) that one launch may take: the last step of the
+    // loop is k1_step's; a mass record reads the height before step t = 0 mod
+    // tdump, a snapshot follows step t = 0 mod snap_every
+    auto steps_at = [&](int64_t it) -> int64_t {
+      int64_t k = std::min<int64_t>(shape.k, nsteps - it);
       const int64_t t = o->t0 + it;
+      auto before = [&](int64_t every, int64_t x) { return every - ((x % every) + every) % every; };
+      if (mass) k = std::min(k, before(p->tdump, t));
+      if (snap) k = std::min(k, before(o->snap_every, t - 1));
+      return k;
+    };
+    for (int64_t it = 1, k; it <= nsteps; it += k) {
+      const int64_t t = o->t0 + it;
+      k = wave ? std::max<int64_t>(1, steps_at(it)) : 1;
       S.h_in = s->hbuf[c];
       S.u_in = s->ubuf[c];
       S.h_out = s->hbuf[1 - c];
@@ -1424,7 +1735,9 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       }
       unsigned long long* kk = keys ? keys + 2 * (it - 1) : nullptr;
       unsigned long long* ww = wet ? wet + (it - 1) : nullptr;
-      if (nbt == 1024)
+      if (wave && it < nsteps)
+        SW_BOTH1(s, launch_wave<T>(S, (uint64_t)t, shape.npt, (int)k, kk, ww, s->stream));
+      else if (nbt == 1024)
         SW_BOTH1(s, hipLaunchKernelGGL((k1_step<T, 1024>), dim3(nb), dim3(1024), 0, s->stream, S,
                                        (uint64_t)t, kk, ww));
       else if (nbt == 512)
@@ -1433,7 +1746,7 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       else
         SW_BOTH1(s, hipLaunchKernelGGL((k1_step<T, 256>), dim3(nb), dim3(256), 0, s->stream, S,
                                        (uint64_t)t, kk, ww));
-      if (snap && t % o->snap_every == 0) {
+      if (snap && (t + k - 1) % o->snap_every == 0) {
         (void)hipMemcpyAsync((char*)snap + ks * s->L * s->esz, S.h_out, s->L * s->esz,
                        hipMemcpyDeviceToDevice, s->stream);
         ++ks;
@@ -1561,14 +1874,15 @@ int swalbe1d_time_loop(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
   (void)hipSetDevice(s->device);
   if (o->variant == 2 && !fits_resident(s, p))
     return bad1("swalbe1d_time_loop: the film does not fit in LDS (variant 2)");
-  const bool resident = o->variant == 2 || (o->variant == 0 && fits_resident(s, p));
+  // `threads` asks for one of the two kernels that take it
+  const bool resident = o->variant == 2 || (o->variant == 0 && o->threads && fits_resident(s, p));
   int rc;
   if (resident) {
     rc = loop_resident(&s, 1, p, nsteps, &o, s->stream, nullptr);
   } else {
     if (o->use_theta_field)
       if ((rc = refresh_kappa(s, p->n, p->m, p->hmin))) return rc;
-    rc = loop_per_step(s, p, nsteps, o);
+    rc = loop_per_step(s, p, nsteps, o, o->variant == 0 && !o->threads);
   }
   if (rc == SWALBE_OK && o->materialize && nsteps > 0) {
     materialize(s, p, o, nsteps);
