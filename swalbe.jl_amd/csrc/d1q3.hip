@@ -53,6 +53,25 @@ __device__ __forceinline__ T powbroad(T a, int n) {
   return r;
 }
 
+// The (n, m) law in the state form: power_broad's products in its order (1 a
+// = a is exact, and the m factors are the first m of the n); the two usual
+// pairs need no loop.  A loop over a run-time n costs a branch per product:
+// 1000 steps of 512 resident films of 1024 nodes took 3.43 ms with the loops,
+// 3.06 without.
+template <typename T>
+__device__ __forceinline__ T disjoin_law(T a, int n, int m) {
+  if (n == 9 && m == 3) {
+    const T a3 = (a * a) * a;
+    const T a6 = ((a3 * a) * a) * a;
+    return (((a6 * a) * a) * a) - a3;
+  }
+  if (n == 3 && m == 2) {
+    const T a2 = a * a;
+    return a2 * a - a2;
+  }
+  return powbroad(a, n) - powbroad(a, m);
+}
+
 // the (n, m) law: power_broad (state form) or fast_93 / fast_32 (raw form),
 // src/pressure.jl:363-422
 template <typename T>
@@ -64,7 +83,7 @@ __device__ __forceinline__ T disjoin(T a, int n, int m, int raw) {
     }
     return ((a * a) * a) - (a * a);
   }
-  return powbroad(a, n) - powbroad(a, m);
+  return disjoin_law(a, n, m);
 }
 
 // p = -γ κ [x^n - x^m] - γ (h[x-1] - 2h + h[x+1]),  x = hmin / (h + hcrit)
@@ -274,8 +293,13 @@ struct Film1 {
   void* u_out;
   void* f_out;
   void* p_out;
-  void* h_last;  // k1_resident: receives the last step's input moments
+  void* h_last;  // the last step's input moments (k1_resident writes them there)
   void* u_last;
+  void* hgp;     // k1_materialize: the last step's intermediates
+  void* slip;
+  void* kbt;
+  void* F;
+  void* feq;
   double* dh;    // k1_resident series: [nsteps], [nsteps], [nmass], [nsnap * L]
   double* wet;
   double* mass;
@@ -285,7 +309,7 @@ struct Film1 {
   uint64_t seed;
   int64_t t0, tdump, snap_every;
   int64_t mass_phase, snap_phase;  // steps before the first mass / snapshot step
-  int L, n, m, thermal, body, read_ft, gg_sign;
+  int L, n, m, thermal, body, read_ft, gg_sign, materialize;
 };
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -423,23 +447,6 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step,
 template <typename T>
 __device__ __forceinline__ __attribute__((address_space(1))) T* glb(T* p) {
   return (__attribute__((address_space(1))) T*)p;
-}
-
-// The (n, m) law of the fused steps: power_broad's products in its order
-// (1 a = a is exact, and the m factors are the first m of the n); the two
-// usual pairs need no loop.
-template <typename T>
-__device__ __forceinline__ T disjoin_law(T a, int n, int m) {
-  if (n == 9 && m == 3) {
-    const T a3 = (a * a) * a;
-    const T a6 = ((a3 * a) * a) * a;
-    return (((a6 * a) * a) * a) - a3;
-  }
-  if (n == 3 && m == 2) {
-    const T a2 = a * a;
-    return a2 * a - a2;
-  }
-  return powbroad(a, n) - powbroad(a, m);
 }
 
 // The value of the lane below / above (DPP wave_shr:1 / wave_shl:1; 0 beyond
@@ -883,6 +890,50 @@ void k1_resident(const Film1* table, int64_t nsteps) {
   }
 }
 
+// The intermediates of a film's last step (h∇p, slip, noise, F, feq) from its
+// input moments and its pressure, each in its per-op kernel's order: films
+// blockIdx.x of the table, in one launch for all of an ensemble (six launches
+// and a synchronisation per film took 17 ms for 512 films, five times the
+// 1000 steps before them).
+template <typename T>
+__device__ __forceinline__ void materialize_node(const Film1& S, uint64_t step, int x) {
+  const int L = S.L;
+  const T* p = (const T*)S.p_out;
+  const int xm = x == 0 ? L - 1 : x - 1, xp = x == L - 1 ? 0 : x + 1;
+  const T hh = ((const T*)S.h_last)[x], u = ((const T*)S.u_last)[x];
+  const T hgp = (hh * T(-0.5)) * (p[xm] - p[xp]);
+  const T sl = slip_node(hh, u, (T)S.c6mu, (T)S.c6d, (T)S.c3dd);
+  ((T*)S.hgp)[x] = hgp;
+  ((T*)S.slip)[x] = sl;
+  T F = -hgp - sl;
+  if (S.thermal) {
+    const T kb = noise_node<T>(S.seed, step, x) * noise_amp(hh, (T)S.kb26, (T)S.delta);
+    ((T*)S.kbt)[x] = kb;
+    F = F - kb;
+  }
+  if (S.gg) {
+    const T gv = ((const T*)S.gg)[x];
+    F = S.gg_sign < 0 ? F - gv : F + gv;
+  }
+  if (S.body) F = F + (hh * (T)S.alpha) * (T)S.fac;
+  ((T*)S.F)[x] = F;
+  T* feq = (T*)S.feq;
+  feq_node(hh, u, (T)S.g, feq[x], feq[L + (int64_t)x], feq[2 * (int64_t)L + x]);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kNT1) void k1_materialize(Film1 S, uint64_t step) {
+  FOR_NODES(x, S.L) materialize_node<T>(S, step, x);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kNT1) void k1_materialize_all(const Film1* table, int64_t nsteps) {
+  const Film1& S = table[blockIdx.x];
+  if (!S.materialize) return;
+  for (int x = blockIdx.y * kNT1 + threadIdx.x; x < S.L; x += gridDim.y * kNT1)
+    materialize_node<T>(S, (uint64_t)(S.t0 + nsteps), x);
+}
+
 // Nodes of a 1D film that one workgroup of k1_reduce folds (at most 256
 // workgroups).  One workgroup for the whole film read L = 3e6 nodes in 4 ms;
 // 256 of them and the finishing wave take 22 us.
@@ -978,6 +1029,9 @@ struct swalbe_film1d {
   void *border[2] = {nullptr, nullptr}, *interior = nullptr;
   bool have_border = false;
   double* red = nullptr;  // 4 doubles, then 4 per workgroup of k1_reduce
+  // film table of the ensembles this film was listed first in
+  Film1* table = nullptr;
+  int table_films = 0;
 };
 
 namespace {
@@ -1202,6 +1256,12 @@ Film1 describe(swalbe_film1d* s, const swalbe_params* p, const swalbe1d_step_opt
   S.ft = s->f[s->ftemp_buf];
   S.f_out = s->f[1 - s->ftemp_buf];
   S.p_out = s->pressure;
+  S.hgp = s->hgp;
+  S.slip = s->slip;
+  S.kbt = s->kbt;
+  S.F = s->F;
+  S.feq = s->feq;
+  S.materialize = o->materialize;
   return S;
 }
 
@@ -1273,7 +1333,7 @@ int swalbe1d_destroy(swalbe_film1d* s) {
   // with other films: this waits for theirs too)
   if (e == hipSuccess && s->stream) e = hipStreamSynchronize(s->stream);
   void* ptrs[] = {s->slab, s->theta, s->kap, s->gamma, s->grad_gamma, s->border[0],
-                  s->border[1], s->interior};
+                  s->border[1], s->interior, s->table};
   for (void* p : ptrs)
     if (p) {
       const hipError_t ef = hipFree(p);
@@ -1501,23 +1561,16 @@ int swalbe1d_resident_max_length(int32_t dtype, int32_t tau_is_one, int32_t* L) 
 
 namespace {
 
-// the intermediates of the last step (pressure, h∇p, slip, noise, F, feq)
-// recomputed by the per-op kernels from its input moments, which the fused
-// loops leave in the other moment buffers
+// The intermediates of the last step of a loop of nsteps > 0 steps, from its
+// input moments (which the fused loops leave in the other moment buffers) and
+// its pressure.
 void materialize(swalbe_film1d* s, const swalbe_params* p, const swalbe1d_step_opts* o,
                  int64_t nsteps) {
-  const int keep = s->cur;
-  s->cur = 1 - s->cur;
-  swalbe1d_filmpressure(s, p->gamma, p->theta, p->n, p->m, p->hmin, p->hcrit,
-                        o->use_theta_field, o->use_gamma_field, 0);
-  swalbe1d_hgradp(s);
-  swalbe1d_slippage(s, p->delta, p->mu);
-  if (o->thermal)
-    swalbe1d_thermal(s, p->kbt, p->mu, p->delta, o->seed, (uint64_t)(o->t0 + nsteps));
-  swalbe1d_force_sum(s, o->thermal, o->grad_gamma);
-  if (o->body) swalbe1d_inclination(s, o->alpha, o->body_fac);
-  swalbe1d_equilibrium(s, p->g);
-  s->cur = keep;
+  Film1 S = describe(s, p, o);
+  S.h_last = s->hbuf[1 - s->cur];
+  S.u_last = s->ubuf[1 - s->cur];
+  SW_BOTH1(s, hipLaunchKernelGGL(k1_materialize<T>, dim3(blocks1d(s->L)), dim3(kNT1), 0,
+                                 s->stream, S, (uint64_t)(o->t0 + nsteps)));
 }
 
 // Device buffers of one film's series (k1_resident writes them directly).
@@ -1542,6 +1595,7 @@ struct Series1 {
   }
   hipError_t fetch(swalbe_film1d* s, const swalbe1d_step_opts* o, hipStream_t st) {
     hipError_t e = hipSuccess;
+    if (!dh && !wet && !mass && !snap) return e;
     std::vector<double> w;
     if (dh) e = hipMemcpyAsync(o->dh_series, dh, 8 * nsteps, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess && wet) {
@@ -1805,6 +1859,7 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
                   double* ms_out) {
   std::vector<Film1> table(nfilms);
   std::vector<Series1> series(nfilms);
+  std::vector<hipStream_t> waited;
   int64_t lds = 0;
   int maxL = 0;
   int rc = SWALBE_OK;
@@ -1813,8 +1868,10 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
     const swalbe1d_step_opts* o = opts[i];
     if (o->use_theta_field) rc = refresh_kappa(s, params[i].n, params[i].m, params[i].hmin);
     if (rc == SWALBE_OK) rc = series[i].alloc(s, &params[i], o, nsteps);
-    if (rc == SWALBE_OK && hipStreamSynchronize(s->stream) != hipSuccess)
-      rc = bad1("swalbe1d: stream error before the resident loop");
+    // work on the films' own streams (a few, shared) comes before the launch
+    if (rc == SWALBE_OK && s->stream != st &&
+        std::find(waited.begin(), waited.end(), s->stream) == waited.end())
+      waited.push_back(s->stream);
     if (rc != SWALBE_OK) break;
     table[i] = describe(s, &params[i], o);
     table[i].dh = series[i].dh;
@@ -1824,10 +1881,21 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
     lds = std::max(lds, resident_bytes(s->L, s->esz, table[i].read_ft));
     maxL = std::max(maxL, s->L);
   }
-  Film1* d_table = nullptr;
+  for (hipStream_t w : waited)
+    if (rc == SWALBE_OK && hipStreamSynchronize(w) != hipSuccess)
+      rc = bad1("swalbe1d: stream error before the resident loop");
   hipError_t e = hipSuccess;
   if (rc == SWALBE_OK && nsteps > 0) {
-    e = hipMalloc(&d_table, sizeof(Film1) * nfilms);
+    swalbe_film1d* own = films[0];
+    if (own->table_films < nfilms) {
+      if (own->table) (void)hipFree(own->table);
+      own->table = nullptr;
+      own->table_films = 0;
+      e = hipMalloc(&own->table, sizeof(Film1) * nfilms);
+      if (e == hipSuccess) own->table_films = nfilms;
+      else own->table = nullptr;
+    }
+    Film1* const d_table = own->table;
     if (e == hipSuccess)
       e = hipMemcpyAsync(d_table, table.data(), sizeof(Film1) * nfilms, hipMemcpyHostToDevice, st);
     const int nt = resident_threads(opts[0]->threads, maxL, nfilms, films[0]->device);
@@ -1841,6 +1909,16 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
       e = films[0]->esz == 8 ? launch_resident<double>(d_table, nfilms, nsteps, lds, nt, st)
                              : launch_resident<float>(d_table, nfilms, nsteps, lds, nt, st);
     if (e == hipSuccess && ms_out) e = hipEventRecord(ev[1], st);
+    bool any = false;
+    for (int i = 0; i < nfilms; ++i) any = any || table[i].materialize;
+    if (e == hipSuccess && any) {
+      const dim3 grid(nfilms, blocks1d(maxL));
+      if (films[0]->esz == 8)
+        hipLaunchKernelGGL(k1_materialize_all<double>, grid, dim3(kNT1), 0, st, d_table, nsteps);
+      else
+        hipLaunchKernelGGL(k1_materialize_all<float>, grid, dim3(kNT1), 0, st, d_table, nsteps);
+      e = hipGetLastError();
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e == hipSuccess && ms_out) {
       float ms = 0.f;
@@ -1855,7 +1933,6 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
     }
   }
   for (auto& sr : series) sr.release();
-  if (d_table) (void)hipFree(d_table);
   if (rc != SWALBE_OK) return rc;
   if (e != hipSuccess) return hip_fail(e, "swalbe1d resident loop");
   return SWALBE_OK;
@@ -1884,7 +1961,7 @@ int swalbe1d_time_loop(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       if ((rc = refresh_kappa(s, p->n, p->m, p->hmin))) return rc;
     rc = loop_per_step(s, p, nsteps, o, o->variant == 0 && !o->threads);
   }
-  if (rc == SWALBE_OK && o->materialize && nsteps > 0) {
+  if (rc == SWALBE_OK && o->materialize && nsteps > 0 && !resident) {
     materialize(s, p, o, nsteps);
     hipError_t e = hipStreamSynchronize(s->stream);
     if (e != hipSuccess) return hip_fail(e, "swalbe1d_time_loop (materialize)");
@@ -1917,14 +1994,7 @@ int swalbe1d_ensemble_time_loop_timed(swalbe_film1d* const* films, int32_t nfilm
       return bad1("swalbe1d_ensemble_time_loop: a film is listed twice");
   }
   (void)hipSetDevice(films[0]->device);
-  int rc = loop_resident(films, nfilms, params, nsteps, po.data(), films[0]->stream, ms_out);
-  for (int i = 0; i < nfilms && rc == SWALBE_OK; ++i)
-    if (po[i]->materialize && nsteps > 0) {
-      materialize(films[i], &params[i], po[i], nsteps);
-      if (hipStreamSynchronize(films[i]->stream) != hipSuccess)
-        rc = bad1("swalbe1d_ensemble_time_loop: materialize failed");
-    }
-  return rc;
+  return loop_resident(films, nfilms, params, nsteps, po.data(), films[0]->stream, ms_out);
 }
 
 int swalbe1d_ensemble_time_loop(swalbe_film1d* const* films, int32_t nfilms,

@@ -95,3 +95,23 @@ def test_fp32_equals_one_launch_per_step(S, name):
         got.append([st.get(k) for k in ("height", "vel", "fout", "pressure")])
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def test_ensemble_intermediates_equal_each_film_alone(S):
+    """One launch writes the last step's intermediates of every film of an ensemble (longer and
+    shorter than a workgroup, with noise, walls, ∇γ, τ ≠ 1; one film without them)."""
+    specs = [(300, "thermal"), (77, "walls"), (700, "gamma_minus"), (256, "tau"), (16, "plain")]
+    n, films, alone = 40, [], []
+    for L, name in specs:
+        for keep in (films, alone):
+            sysc, prm, st, ost, okw, hkw, args = _setup(S, L, n, CONFIGS[name])
+            keep.append((sysc, st, hkw))
+    for sysc, st, hkw in alone:
+        S.time_loop(sysc, st, **hkw)
+    S.ensemble_time_loop([f[0] for f in films], [f[1] for f in films], n,
+                         thermal=[f[2]["thermal"] for f in films], seed=11,
+                         γ=[f[2].get("γ") for f in films],
+                         grad_gamma_sign=[f[2].get("grad_gamma_sign", 0) for f in films])
+    for (_, a, _), (_, b, _), spec in zip(films, alone, specs):
+        for name in ("height", "vel", "fout", "pressure", "hgradp", "slip", "kbt", "F", "feq"):
+            assert np.array_equal(a.get(name), b.get(name)), (spec, name)
