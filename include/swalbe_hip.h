@@ -157,7 +157,9 @@ typedef struct swalbe_step_opts {
     int32_t tile_y;        /* rows per workgroup tile: 0 = default (16 for FP32; FP64 16 where
                               h, ux, uy exceed 32 MB, else 8);
                               8 or 16 (the same results either way); variant 3: rows per
-                              strip segment, 0 = default (64), 4..4096 */
+                              strip segment, 0 = default (64), 4..4096.  With tile_y = 0 and
+                              variant = 0 small films take several steps per launch, and
+                              only the last step writes the distributions and the pressure */
     int32_t variant;       /* FP32 kernel: 0 = default (2), 1 = LDS tiles, collide at the
                               source node, 2 = LDS tiles, collide at the destination node,
                               3 = LDS-free strips (one wavefront per 58-column strip) */

@@ -827,9 +827,10 @@ struct LoopBuffers {
   }
 };
 
+// `multi`: nsub steps from t in one launch of its shape (geom >= 0).
 template <typename T>
 void enqueue_step(swalbe_state* st, const StepParams& sp, StepSeries ser, uint64_t t, int tile_y,
-                  int variant, int nts, bool outs) {
+                  int variant, int nts, bool outs, const MultiShape& multi, int nsub) {
   Film& F = st->film;
   const int cur = F.hu_cur;
   const int fdst = F.fout_buf != F.ftemp_buf ? F.fout_buf : 1 - F.ftemp_buf;
@@ -844,6 +845,13 @@ void enqueue_step(swalbe_state* st, const StepParams& sp, StepSeries ser, uint64
   io.uy_out = (T*)F.uybuf[1 - cur];
   io.p_out = (T*)F.pressure;
   io.kappa = sp.use_theta ? (const T*)F.kappa : nullptr;
+  if (multi.geom >= 0) {
+    launch_multi<T>(io, sp, ser, t, nsub, outs, F.Lx, F.Ly, F.fstride, F.enc, multi.geom,
+                    st->stream);
+    F.fout_buf = F.ftemp_buf = fdst;
+    F.hu_cur = 1 - cur;
+    return;
+  }
   if (!outs) {  // distributions and pressure of a step nobody reads (τ = 1)
     io.f_out = nullptr;
     io.p_out = nullptr;
@@ -998,8 +1006,25 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
     SW_HIP(hipEventRecord(e0, st->stream));
   }
   int64_t km = 0;
-  for (int64_t it = 1; it <= nsteps; ++it) {
+  // Small films take several steps per launch.  The loop's last step is a
+  // launch of its own (its input moments stay in the other buffer for
+  // materialize_last), and so is every step that something falls between:
+  // a mass record or a measurement before step t, a snapshot after it.
+  const bool automatic = o->variant == 0 && o->tile_y <= 0;
+  const MultiShape multi = automatic ? multi_shape(F.Lx, F.Ly, F.dtype == SWALBE_F64)
+                                     : MultiShape{-1, 1};
+  auto steps_at = [&](int64_t it) -> int64_t {
+    if (multi.geom < 0 || want_meas) return 1;
+    int64_t k = std::min<int64_t>(multi.k, nsteps - it);
     const int64_t t = o->t0 + it;
+    auto before = [](int64_t every, int64_t x) { return every - ((x % every) + every) % every; };
+    if (want_mass) k = std::min(k, before(p->tdump, t));
+    if (want_snap) k = std::min(k, before(o->snap_every, t - 1));
+    return std::max<int64_t>(k, 1);
+  };
+  for (int64_t it = 1, nsub = 1; it <= nsteps; it += nsub) {
+    const int64_t t = o->t0 + it;
+    nsub = steps_at(it);
     if (want_mass && t % p->tdump == 0) {
       if (int rc = reduce_enqueue(st, F.height(), enc_offset(F, SWALBE_HEIGHT, 0), 0.0,
                                   lb.mass + 4 * km))
@@ -1015,12 +1040,14 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
                       st->nparts, lb.meas + 4 * (it - 1), st->stream));
     }
     StepSeries ser{want_dh ? lb.keys + 2 * (it - 1) : nullptr, want_wet ? lb.wet + (it - 1) : nullptr};
-    const bool outs = !final_only || it == nsteps;
+    const bool outs = multi.geom >= 0 ? it == nsteps : !final_only || it == nsteps;
     if (F.dtype == SWALBE_F64)
-      enqueue_step<double>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs);
+      enqueue_step<double>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
+                           multi, (int)nsub);
     else
-      enqueue_step<float>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs);
-    if (want_snap && t % o->snap_every == 0) {
+      enqueue_step<float>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
+                           multi, (int)nsub);
+    if (want_snap && (t + nsub - 1) % o->snap_every == 0) {
       const int r = (int)(ksnap % SnapRing::R);
       if (int rc = snap_drain(r)) return rc;
       SW_HIP(hipMemcpyAsync(ring.dev[r], F.height(), plane_bytes, hipMemcpyDeviceToDevice,

@@ -16,6 +16,7 @@
 // FP64: every value equals the unfused reference sequence bit for bit (same
 // expressions, same order, no contraction).  FP32: height and distributions
 // are handled as deviations from a rest film of height href (Enc).
+#include "step_node.h"
 #include "swalbe_internal.h"
 
 namespace swalbe {
@@ -31,37 +32,6 @@ __device__ __forceinline__ int wrap1(int a, int L) {
 __device__ __forceinline__ int wrapm(int a, int L) {
   a %= L;
   return a < 0 ? a + L : a;
-}
-
-template <typename T>
-__device__ __forceinline__ T powlaw(T a, int n, int m, int mode) {
-  if (mode == 1) {
-    const T t = (a * a) * a;
-    return ((t * t) * t) - t;
-  }
-  if (mode == 2) return ((a * a) * a) - (a * a);
-  T tn = T(1), tm = T(1);
-  for (int i = 0; i < n; ++i) tn *= a;
-  for (int i = 0; i < m; ++i) tm *= a;
-  return tn - tm;
-}
-
-// Equilibrium population k at a node (src/equilibrium.jl:71-114), plain values.
-template <typename T>
-__device__ __forceinline__ T feq_k(int k, T h, T u, T v, T usq, T c56g, T g0) {
-  const T w1 = T(1.0 / 9.0), w5 = T(1.0 / 36.0);
-  T a;
-  switch (k) {
-    case 0: return h * ((T(1) - c56g * h) - T(2.0 / 3.0) * usq);
-    case 1: return w1 * h * (((g0 * h + T(3) * u) + T(4.5) * (u * u)) - T(1.5) * usq);
-    case 2: return w1 * h * (((g0 * h + T(3) * v) + T(4.5) * (v * v)) - T(1.5) * usq);
-    case 3: return w1 * h * (((g0 * h - T(3) * u) + T(4.5) * (u * u)) - T(1.5) * usq);
-    case 4: return w1 * h * (((g0 * h - T(3) * v) + T(4.5) * (v * v)) - T(1.5) * usq);
-    case 5: a = u + v; return w5 * h * (((g0 * h + T(3) * a) + T(4.5) * (a * a)) - T(1.5) * usq);
-    case 6: a = v - u; return w5 * h * (((g0 * h + T(3) * a) + T(4.5) * (a * a)) - T(1.5) * usq);
-    case 7: a = u + v; return w5 * h * (((g0 * h - T(3) * a) + T(4.5) * (a * a)) - T(1.5) * usq);
-    default: a = u - v; return w5 * h * (((g0 * h + T(3) * a) + T(4.5) * (a * a)) - T(1.5) * usq);
-  }
 }
 
 // Deviation feq_k(h, u) - feq_k(href, 0) with h = href + dh, free of the
@@ -83,22 +53,6 @@ __device__ __forceinline__ float feq_dev(int k, float dh, float h, float href, f
   }
   const float w = k <= 4 ? (1.0f / 9.0f) : (1.0f / 36.0f);
   return w * (g0 * gg + h * ((s * 3.0f * a + 4.5f * (a * a)) - 1.5f * usq));
-}
-
-template <typename T>
-__device__ __forceinline__ T force_term(int k, T Fx, T Fy) {
-  const T c3 = T(1.0 / 3.0), c24 = T(1.0 / 24.0);
-  switch (k) {
-    case 1: return c3 * Fx;
-    case 2: return c3 * Fy;
-    case 3: return -(c3 * Fx);
-    case 4: return -(c3 * Fy);
-    case 5: return c24 * (Fx + Fy);
-    case 6: return c24 * (Fy - Fx);
-    case 7: return -(c24 * (Fx + Fy));
-    case 8: return c24 * (Fx - Fy);
-    default: return T(0);
-  }
 }
 
 // The force on one node.

@@ -21,6 +21,7 @@
 // a batch.
 #include <type_traits>
 
+#include "step_node.h"
 #include "swalbe_batch.h"
 
 namespace swalbe {
@@ -37,48 +38,6 @@ __device__ __forceinline__ int wrap1(int a, int L) {
 __device__ __forceinline__ int wrapm(int a, int L) {
   a %= L;
   return a < 0 ? a + L : a;
-}
-
-__device__ __forceinline__ float powlaw_f(float a, int n, int m, int mode) {
-  if (mode == 1) {
-    const float t = (a * a) * a;
-    return (t * t - 1.0f) * t;
-  }
-  if (mode == 2) return (a - 1.0f) * (a * a);
-  float tn = 1.0f, tm = 1.0f;
-  for (int i = 0; i < n; ++i) tn *= a;
-  for (int i = 0; i < m; ++i) tm *= a;
-  return tn - tm;
-}
-
-__device__ __forceinline__ double powlaw_d(double a, int n, int m, int mode) {
-  if (mode == 1) {
-    const double t = (a * a) * a;
-    return (t * t - 1.0) * t;
-  }
-  if (mode == 2) return (a - 1.0) * (a * a);
-  double tn = 1.0, tm = 1.0;
-  for (int i = 0; i < n; ++i) tn *= a;
-  for (int i = 0; i < m; ++i) tm *= a;
-  return tn - tm;
-}
-
-// The disjoining part of the film pressure, -γ κ [a^n - a^m] with
-// a = hmin / (h + hcrit), at a node of stored height deviation dh.  Where the
-// film nears hmin (h < hguard) the term dominates the pressure and is
-// evaluated in FP64 from the stored height with an IEEE division; elsewhere
-// in FP32 with v_rcp_f32.  kap is κ (a θ field's value, or the film's).
-__device__ __forceinline__ float disjoining_f(const F32K& K, float dh, float kap, bool kap_field) {
-#pragma clang fp contract(fast)
-  const float hh = K.href + dh;
-  if (K.guard && hh < K.hguard) {
-    const double hd = K.href_d + (double)dh;
-    const double a = K.hmin_d / (hd + K.hcrit_d);
-    const double kd = kap_field ? (double)kap : K.kap_d;
-    return (float)(-K.gamma_d * (kd * powlaw_d(a, K.n, K.m, K.powmode)));
-  }
-  const float a = K.hmin * __builtin_amdgcn_rcpf(hh + K.hcrit);
-  return -K.gamma * (kap * powlaw_f(a, K.n, K.m, K.powmode));
 }
 
 // p, a pointer uniform over the wave, as the compiler's scalar registers hold

@@ -207,6 +207,19 @@ void launch_step_f32(const StepIO<float>& io, const StepParams& sp, StepSeries s
                      int Lx, int Ly, int64_t fstride, Enc enc, int tile_y, int variant, int nts,
                      hipStream_t s);
 
+// Several steps of a small film per launch (step_multi.hip).  The shape for a
+// film, and a launch of k <= shape.k steps; ser: the series slots of the
+// first; write_f: the last of them writes f and p (τ ≠ 1: f always).
+struct MultiShape {
+  int geom;  // -1: one step per launch is the faster path
+  int k;
+};
+MultiShape multi_shape(int Lx, int Ly, bool f64);
+template <typename T>
+void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step, int k,
+                  bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int geom,
+                  hipStream_t s);
+
 // Deterministic FP64 reductions of a field: sum, max, min, count(> thresh).
 template <typename T>
 void launch_reduce(const T* h, int64_t N, double href, double thresh, double* partials,
