@@ -775,20 +775,6 @@ StepParams make_step_params(const swalbe_params* p, const swalbe_step_opts* o, i
 
 namespace {
 
-__global__ void k_fill_u64(unsigned long long* p, unsigned long long v, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = v;
-}
-
-__global__ void k_init_keys(unsigned long long* p, int64_t nsteps) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nsteps;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    p[2 * i] = 0ull;
-    p[2 * i + 1] = ~0ull;
-  }
-}
-
 // Snapshots of the height: a device copy per snapshot into a ring slot on
 // the state's stream, then a device-to-host copy of that slot on a second
 // stream into pinned staging, decoded once the slot comes round again.
@@ -813,14 +799,10 @@ struct SnapRing {
 };
 
 struct LoopBuffers {
-  unsigned long long* keys = nullptr;  // 2 per step
-  unsigned long long* wet = nullptr;   // 1 per step
   double* mass = nullptr;              // 4 per tdump
   double* meas = nullptr;              // 4 per step: count, max, area, energy
   uint8_t* fluid = nullptr;            // Lx*Ly per step
   ~LoopBuffers() {
-    if (keys) hipFree(keys);
-    if (wet) hipFree(wet);
     if (mass) hipFree(mass);
     if (meas) hipFree(meas);
     if (fluid) hipFree(fluid);
@@ -957,15 +939,12 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
   if (want_meas) SW_HIP(hipMalloc((void**)&lb.meas, sizeof(double) * 4 * std::max<int64_t>(1, nsteps)));
   if (want_fluid) SW_HIP(hipMalloc((void**)&lb.fluid, (size_t)F.N * std::max<int64_t>(1, nsteps)));
   const double meas_thresh = o->surf_thresh > 0.0 ? o->surf_thresh : 0.055;
-  if (want_dh) SW_HIP(hipMalloc(&lb.keys, sizeof(unsigned long long) * 2 * std::max<int64_t>(1, nsteps)));
-  if (want_wet) SW_HIP(hipMalloc(&lb.wet, sizeof(unsigned long long) * std::max<int64_t>(1, nsteps)));
+  SeriesRun series;
+  SW_HIP(series.start(nsteps, want_dh, want_wet, st->stream));
   int64_t nmass = 0;
   for (int64_t it = 1; it <= nsteps && want_mass; ++it)
     if ((o->t0 + it) % p->tdump == 0) ++nmass;
   if (want_mass && nmass) SW_HIP(hipMalloc(&lb.mass, sizeof(double) * 4 * nmass));
-  if (want_dh)  // even slots hold max keys (start 0), odd slots min keys (start ~0)
-    hipLaunchKernelGGL(k_init_keys, dim3(64), dim3(256), 0, st->stream, lb.keys, nsteps);
-  if (want_wet) hipLaunchKernelGGL(k_fill_u64, dim3(64), dim3(256), 0, st->stream, lb.wet, 0ull, nsteps);
   const bool want_snap = o->snap_every > 0 && o->snap_series != nullptr;
   if (ms_out && want_snap) {
     set_error("swalbe_time_loop_timed: snapshots are not taken by the timed variant");
@@ -1020,6 +999,7 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
     auto before = [](int64_t every, int64_t x) { return every - ((x % every) + every) % every; };
     if (want_mass) k = std::min(k, before(p->tdump, t));
     if (want_snap) k = std::min(k, before(o->snap_every, t - 1));
+    k = std::min(k, series.room(it - 1));
     return std::max<int64_t>(k, 1);
   };
   for (int64_t it = 1, nsub = 1; it <= nsteps; it += nsub) {
@@ -1039,7 +1019,7 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
                       want_fluid ? lb.fluid + (size_t)F.N * (it - 1) : nullptr, st->partials,
                       st->nparts, lb.meas + 4 * (it - 1), st->stream));
     }
-    StepSeries ser{want_dh ? lb.keys + 2 * (it - 1) : nullptr, want_wet ? lb.wet + (it - 1) : nullptr};
+    const StepSeries ser = series.at(it - 1);
     const bool outs = multi.geom >= 0 ? it == nsteps : !final_only || it == nsteps;
     if (F.dtype == SWALBE_F64)
       enqueue_step<double>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
@@ -1047,6 +1027,7 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
     else
       enqueue_step<float>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
                            multi, (int)nsub);
+    series.taken(it - 1, nsub, st->stream);
     if (want_snap && (t + nsub - 1) % o->snap_every == 0) {
       const int r = (int)(ksnap % SnapRing::R);
       if (int rc = snap_drain(r)) return rc;
@@ -1076,13 +1057,13 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
     else materialize_last<float>(st, p, o, (uint64_t)(o->t0 + nsteps));
     SW_HIP(hipGetLastError());
   }
-  if (want_dh) {
-    std::vector<unsigned long long> keys(2 * nsteps);
-    SW_HIP(hipMemcpyAsync(keys.data(), lb.keys, keys.size() * 8, hipMemcpyDeviceToHost, st->stream));
-    SW_HIP(hipStreamSynchronize(st->stream));
+  if (series.on()) {
+    std::vector<double> v(3 * nsteps);  // max, min, count
+    SW_HIP(series.fetch(v.data(), st->stream));
     for (int64_t i = 0; i < nsteps; ++i) {
-      if (o->dh_series) o->dh_series[i] = dkey_inv(keys[2 * i]) - dkey_inv(keys[2 * i + 1]);
-      if (want_maxh) o->maxh_series[i] = dkey_inv(keys[2 * i]);
+      if (o->dh_series) o->dh_series[i] = v[3 * i] - v[3 * i + 1];
+      if (want_maxh) o->maxh_series[i] = v[3 * i];
+      if (want_wet) o->wet_series[i] = (int64_t)v[3 * i + 2];
     }
   }
   if (want_meas && nsteps > 0) {
@@ -1096,12 +1077,6 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
       if (o->area_series) o->area_series[i] = m[4 * i + 2];
       if (o->energy_series) o->energy_series[i] = m[4 * i + 3];
     }
-  }
-  if (want_wet) {
-    std::vector<unsigned long long> w(nsteps);
-    SW_HIP(hipMemcpyAsync(w.data(), lb.wet, w.size() * 8, hipMemcpyDeviceToHost, st->stream));
-    SW_HIP(hipStreamSynchronize(st->stream));
-    for (int64_t i = 0; i < nsteps; ++i) o->wet_series[i] = (int64_t)w[i];
   }
   if (want_mass && nmass) {
     std::vector<double> m(4 * nmass);

@@ -345,9 +345,7 @@ constexpr int k1_npt(int nb) { return nb <= 512 ? 2 : 1; }
 // neither order nor grouping changes a result.
 
 template <typename T, int NB>
-__global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step,
-                                              unsigned long long* dh_keys,
-                                              unsigned long long* wet) {
+__global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step, swalbe::StepSeries ser) {
   constexpr int NPT = k1_npt(NB), W = NB * NPT;
   __shared__ T sh[W + 6], su[W + 2], sp[W + 4], s0[W + 2], s1[W + 2], s2[W + 2];
   const int t = threadIdx.x, L = S.L;
@@ -399,7 +397,7 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step,
     const int j = t + q * NB;  // output node x0 + j
     const int x = x0 + j;
     if (x >= L) break;
-    if (dh_keys || wet) {
+    if (ser.base) {
       const double hv = (double)sh[j + 3];
       const unsigned long long k = dkey(hv);
       kmax = k > kmax ? k : kmax;
@@ -424,20 +422,14 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step,
     ((T*)S.u_out)[x] = (f1 - f2) / hn;
     __builtin_nontemporal_store(sp[j + 2], &((T*)S.p_out)[x]);
   }
-  if (dh_keys || wet) {  // one atomic per wave
+  if (ser.base) {  // one result per wave
     for (int o = 32; o > 0; o >>= 1) {
       const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
       kmax = a > kmax ? a : kmax;
       kmin = b < kmin ? b : kmin;
       cnt += __shfl_xor(cnt, o);
     }
-    if ((t & 63) == 0) {
-      if (dh_keys) {
-        atomicMax(&dh_keys[0], kmax);
-        atomicMin(&dh_keys[1], kmin);
-      }
-      if (wet && cnt) atomicAdd(wet, cnt);
-    }
+    if ((t & 63) == 0) ser.add(0, kmax, kmin, cnt);
   }
 }
 
@@ -494,8 +486,7 @@ __device__ __forceinline__ T from_above(T v) {
 // EXTRA: any of the κ, γ, ∇γ fields or walls; RFT: τ ≠ 1; TH: noise.
 template <typename T, int NPT, bool RFT, bool TH, bool EXTRA>
 __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, int W,
-                                              unsigned long long* dh_keys,
-                                              unsigned long long* wet) {
+                                              swalbe::StepSeries ser) {
   const int lane = threadIdx.x, L = S.L;
   const int64_t x0 = (int64_t)blockIdx.x * W;         // first node written
   const int64_t xs = x0 - 3 * k + (int64_t)lane * NPT;  // this lane's first node
@@ -540,7 +531,7 @@ __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, in
   const int own0 = 3 * k - lane * NPT;  // nodes j with own0 <= j < own0 + W are this wave's
 #pragma unroll 1
   for (int s = 0; s < k; ++s) {
-    if (dh_keys || wet) {  // series over the step's input height
+    if (ser.base) {  // series over the step's input height
       unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
 #pragma unroll
       for (int j = 0; j < NPT; ++j)
@@ -557,13 +548,7 @@ __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, in
         kmin = b < kmin ? b : kmin;
         cnt += __shfl_xor(cnt, o);
       }
-      if (lane == 0) {
-        if (dh_keys) {
-          atomicMax(&dh_keys[2 * s], kmax);
-          atomicMin(&dh_keys[2 * s + 1], kmin);
-        }
-        if (wet && cnt) atomicAdd(&wet[s], cnt);
-      }
+      if (lane == 0) ser.add(s, kmax, kmin, cnt);
     }
     T p[NPT];
     {
@@ -993,20 +978,6 @@ void launch_reduce1(const T* h, const T* inter, int L, double thresh, double* pa
   hipLaunchKernelGGL(k1_reduce<T>, dim3(nb), dim3(256), 0, st, h, inter, L, thresh,
                      nb == 1 ? out : parts);
   if (nb > 1) swalbe::launch_reduce_finish(parts, nb, out, st);
-}
-
-__global__ void k1_init_keys(unsigned long long* k, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    k[2 * i] = 0ull;
-    k[2 * i + 1] = ~0ull;
-  }
-}
-
-__global__ void k1_zero_u64(unsigned long long* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0ull;
 }
 
 }  // namespace
@@ -1696,41 +1667,41 @@ WaveShape wave_shape(int L, int most, int simds) {
 }
 
 template <typename T, int NPT, bool RFT, bool TH, bool EXTRA>
-void launch_wave_t(const Film1& S, uint64_t step, int k, unsigned long long* kk,
-                   unsigned long long* ww, hipStream_t st) {
+void launch_wave_t(const Film1& S, uint64_t step, int k, swalbe::StepSeries ser,
+                   hipStream_t st) {
   const int W = 64 * NPT - 6 * k;
   hipLaunchKernelGGL((k1_wave<T, NPT, RFT, TH, EXTRA>), dim3((S.L - 1) / W + 1), dim3(64), 0, st,
-                     S, step, k, W, kk, ww);
+                     S, step, k, W, ser);
 }
 
 template <typename T, int NPT>
-void launch_wave_n(const Film1& S, uint64_t step, int k, unsigned long long* kk,
-                   unsigned long long* ww, hipStream_t st) {
+void launch_wave_n(const Film1& S, uint64_t step, int k, swalbe::StepSeries ser,
+                   hipStream_t st) {
   const bool extra = S.kap || S.gam || S.gg || S.b1;
   if (S.read_ft) {
     if (S.thermal)
-      extra ? launch_wave_t<T, NPT, true, true, true>(S, step, k, kk, ww, st)
-            : launch_wave_t<T, NPT, true, true, false>(S, step, k, kk, ww, st);
+      extra ? launch_wave_t<T, NPT, true, true, true>(S, step, k, ser, st)
+            : launch_wave_t<T, NPT, true, true, false>(S, step, k, ser, st);
     else
-      extra ? launch_wave_t<T, NPT, true, false, true>(S, step, k, kk, ww, st)
-            : launch_wave_t<T, NPT, true, false, false>(S, step, k, kk, ww, st);
+      extra ? launch_wave_t<T, NPT, true, false, true>(S, step, k, ser, st)
+            : launch_wave_t<T, NPT, true, false, false>(S, step, k, ser, st);
   } else if (S.thermal) {
-    extra ? launch_wave_t<T, NPT, false, true, true>(S, step, k, kk, ww, st)
-          : launch_wave_t<T, NPT, false, true, false>(S, step, k, kk, ww, st);
+    extra ? launch_wave_t<T, NPT, false, true, true>(S, step, k, ser, st)
+          : launch_wave_t<T, NPT, false, true, false>(S, step, k, ser, st);
   } else {
-    extra ? launch_wave_t<T, NPT, false, false, true>(S, step, k, kk, ww, st)
-          : launch_wave_t<T, NPT, false, false, false>(S, step, k, kk, ww, st);
+    extra ? launch_wave_t<T, NPT, false, false, true>(S, step, k, ser, st)
+          : launch_wave_t<T, NPT, false, false, false>(S, step, k, ser, st);
   }
 }
 
-// k steps of k1_wave; kk, ww: the series slots of its first step
+// k steps of k1_wave; ser: the series slots of its first step
 template <typename T>
-void launch_wave(const Film1& S, uint64_t step, int npt, int k, unsigned long long* kk,
-                 unsigned long long* ww, hipStream_t st) {
-  if (npt == 8) launch_wave_t<T, 8, false, false, false>(S, step, k, kk, ww, st);
-  else if (npt == 4) launch_wave_n<T, 4>(S, step, k, kk, ww, st);
-  else if (npt == 2) launch_wave_n<T, 2>(S, step, k, kk, ww, st);
-  else launch_wave_n<T, 1>(S, step, k, kk, ww, st);
+void launch_wave(const Film1& S, uint64_t step, int npt, int k, swalbe::StepSeries ser,
+                 hipStream_t st) {
+  if (npt == 8) launch_wave_t<T, 8, false, false, false>(S, step, k, ser, st);
+  else if (npt == 4) launch_wave_n<T, 4>(S, step, k, ser, st);
+  else if (npt == 2) launch_wave_n<T, 2>(S, step, k, ser, st);
+  else launch_wave_n<T, 1>(S, step, k, ser, st);
 }
 
 // The loop in launches of k1_step (any L) or, with `wave`, of k1_wave for
@@ -1739,21 +1710,17 @@ void launch_wave(const Film1& S, uint64_t step, int npt, int k, unsigned long lo
 // buffers of each
 int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
                   const swalbe1d_step_opts* o, bool wave) {
-  unsigned long long *keys = nullptr, *wet = nullptr;
+  swalbe::SeriesRun series;
   double* mass = nullptr;
   void* snap = nullptr;
   const int64_t nmass = o->mass_series ? count_every(o->t0, nsteps, p->tdump) : 0;
   const int64_t nsnap = o->snap_series ? count_every(o->t0, nsteps, o->snap_every) : 0;
-  const int64_t ns = std::max<int64_t>(1, nsteps);
   bool ok = true;
-  if (o->dh_series) ok = ok && hipMalloc(&keys, 16 * ns) == hipSuccess;
-  if (o->wet_series) ok = ok && hipMalloc(&wet, 8 * ns) == hipSuccess;
+  ok = series.start(nsteps, o->dh_series, o->wet_series, s->stream) == hipSuccess;
   if (nmass) ok = ok && hipMalloc(&mass, 32 * nmass) == hipSuccess;
   if (nsnap) ok = ok && hipMalloc(&snap, (size_t)nsnap * s->L * s->esz) == hipSuccess;
   hipError_t e = hipSuccess;
   if (ok) {
-    if (keys) hipLaunchKernelGGL(k1_init_keys, dim3(64), dim3(256), 0, s->stream, keys, ns);
-    if (wet) hipLaunchKernelGGL(k1_zero_u64, dim3(64), dim3(256), 0, s->stream, wet, ns);
     Film1 S = describe(s, p, o);
     int a = s->ftemp_buf, c = s->cur;
     int64_t km = 0, ks = 0;
@@ -1771,6 +1738,7 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       auto before = [&](int64_t every, int64_t x) { return every - ((x % every) + every) % every; };
       if (mass) k = std::min(k, before(p->tdump, t));
       if (snap) k = std::min(k, before(o->snap_every, t - 1));
+      k = std::min(k, series.room(it - 1));
       return k;
     };
     for (int64_t it = 1, k; it <= nsteps; it += k) {
@@ -1787,19 +1755,19 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
                                    mass + 4 * km, s->stream));
         ++km;
       }
-      unsigned long long* kk = keys ? keys + 2 * (it - 1) : nullptr;
-      unsigned long long* ww = wet ? wet + (it - 1) : nullptr;
+      const swalbe::StepSeries ser = series.at(it - 1);
       if (wave && it < nsteps)
-        SW_BOTH1(s, launch_wave<T>(S, (uint64_t)t, shape.npt, (int)k, kk, ww, s->stream));
+        SW_BOTH1(s, launch_wave<T>(S, (uint64_t)t, shape.npt, (int)k, ser, s->stream));
       else if (nbt == 1024)
         SW_BOTH1(s, hipLaunchKernelGGL((k1_step<T, 1024>), dim3(nb), dim3(1024), 0, s->stream, S,
-                                       (uint64_t)t, kk, ww));
+                                       (uint64_t)t, ser));
       else if (nbt == 512)
         SW_BOTH1(s, hipLaunchKernelGGL((k1_step<T, 512>), dim3(nb), dim3(512), 0, s->stream, S,
-                                       (uint64_t)t, kk, ww));
+                                       (uint64_t)t, ser));
       else
         SW_BOTH1(s, hipLaunchKernelGGL((k1_step<T, 256>), dim3(nb), dim3(256), 0, s->stream, S,
-                                       (uint64_t)t, kk, ww));
+                                       (uint64_t)t, ser));
+      series.taken(it - 1, k, s->stream);
       if (snap && (t + k - 1) % o->snap_every == 0) {
         (void)hipMemcpyAsync((char*)snap + ks * s->L * s->esz, S.h_out, s->L * s->esz,
                        hipMemcpyDeviceToDevice, s->stream);
@@ -1813,18 +1781,13 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
       s->cur = c;
     }
     e = hipGetLastError();
-    if (e == hipSuccess && keys) {
-      std::vector<unsigned long long> k(2 * nsteps);
-      e = hipMemcpyAsync(k.data(), keys, k.size() * 8, hipMemcpyDeviceToHost, s->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-      for (int64_t i = 0; i < nsteps && e == hipSuccess; ++i)
-        o->dh_series[i] = dkey_inv(k[2 * i]) - dkey_inv(k[2 * i + 1]);
-    }
-    if (e == hipSuccess && wet) {
-      std::vector<unsigned long long> w(nsteps);
-      e = hipMemcpyAsync(w.data(), wet, w.size() * 8, hipMemcpyDeviceToHost, s->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-      for (int64_t i = 0; i < nsteps && e == hipSuccess; ++i) o->wet_series[i] = (int64_t)w[i];
+    if (e == hipSuccess && series.on()) {
+      std::vector<double> v(3 * nsteps);  // max, min, count
+      e = series.fetch(v.data(), s->stream);
+      for (int64_t i = 0; i < nsteps && e == hipSuccess; ++i) {
+        if (o->dh_series) o->dh_series[i] = v[3 * i] - v[3 * i + 1];
+        if (o->wet_series) o->wet_series[i] = (int64_t)v[3 * i + 2];
+      }
     }
     if (e == hipSuccess && mass) {
       std::vector<double> mm(4 * nmass);
@@ -1844,8 +1807,6 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
     set_error("swalbe1d_time_loop: allocation of the series failed");
   }
   (void)hipStreamSynchronize(s->stream);
-  if (keys) (void)hipFree(keys);
-  if (wet) (void)hipFree(wet);
   if (mass) (void)hipFree(mass);
   if (snap) (void)hipFree(snap);
   if (!ok) return SWALBE_ENOMEM;

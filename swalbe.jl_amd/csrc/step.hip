@@ -407,7 +407,7 @@ __global__ __launch_bounds__(NT) void k_step(StepIO<T> io, StepParams sp, StepSe
     if constexpr (!AL) {
       if (io.p_out) store_t<NTS != 0>(at(io.p_out, lane_off()), sh_p[(row + 2) * PC + (tx + 2)]);
     }
-    if (ser.dh_keys || ser.wet) {
+    if (ser.base) {
       const T hc = sh_h[(row + 3) * HC + (tx + 3)];
       const double hv = DEV ? (double)href + (double)hc : (double)hc;
       lmax = hv > lmax ? hv : lmax;
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(NT) void k_step(StepIO<T> io, StepParams sp, StepSe
 
   __builtin_amdgcn_s_setprio(0);
   // ---- per-step series: max/min/count of h_t over the domain (exact)
-  if (ser.dh_keys || ser.wet) {
+  if (ser.base) {
     unsigned long long kmax = dkey(lmax), kmin = dkey(lmin);
     for (int o = 32; o > 0; o >>= 1) {
       const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
@@ -438,11 +438,7 @@ __global__ __launch_bounds__(NT) void k_step(StepIO<T> io, StepParams sp, StepSe
         kmin = red_k[2 * w + 1] < kmin ? red_k[2 * w + 1] : kmin;
         lcnt += red_c[w];
       }
-      if (ser.dh_keys) {
-        atomicMax(&ser.dh_keys[0], kmax);
-        atomicMin(&ser.dh_keys[1], kmin);
-      }
-      if (ser.wet) atomicAdd(&ser.wet[0], (unsigned long long)lcnt);
+      ser.add(0, kmax, kmin, lcnt);
     }
   }
 }
@@ -483,6 +479,45 @@ void launch_ty(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64
   }
 #undef SW_M
 #undef SW_K
+}
+
+// ---------------------------------------------------------------- series
+// slots of n steps to their neutral values
+__global__ void k_series_init(unsigned long long* slots, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n * kSeriesSlots;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    unsigned long long* s = slots + i * kSeriesWords;
+    s[0] = 0ull;
+    s[1] = ~0ull;
+    s[2] = 0ull;
+  }
+}
+
+// one wave per step: folds the step's slots and makes them neutral again
+__global__ __launch_bounds__(64) void k_series_fold(unsigned long long* slots, double* out) {
+  static_assert(kSeriesSlots <= 64, "one slot per lane");
+  unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
+  if (threadIdx.x < kSeriesSlots) {
+    unsigned long long* s =
+        slots + ((int64_t)blockIdx.x * kSeriesSlots + threadIdx.x) * kSeriesWords;
+    kmax = s[0];
+    kmin = s[1];
+    cnt = s[2];
+    s[0] = 0ull;
+    s[1] = ~0ull;
+    s[2] = 0ull;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
+    kmax = a > kmax ? a : kmax;
+    kmin = b < kmin ? b : kmin;
+    cnt += __shfl_xor(cnt, o);
+  }
+  if (threadIdx.x == 0) {
+    out[3 * (int64_t)blockIdx.x] = dkey_inv(kmax);
+    out[3 * (int64_t)blockIdx.x + 1] = dkey_inv(kmin);
+    out[3 * (int64_t)blockIdx.x + 2] = (double)cnt;
+  }
 }
 
 // ---------------------------------------------------------------- reductions
@@ -582,6 +617,40 @@ void launch_reduce(const T* h, int64_t N, double href, double thresh, double* pa
 
 void launch_reduce_finish(const double* partials, int nparts, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, partials, nparts, out);
+}
+
+SeriesRun::~SeriesRun() {
+  if (slots) (void)hipFree(slots);
+  if (folded) (void)hipFree(folded);
+}
+
+hipError_t SeriesRun::start(int64_t n, bool want_dh, bool want_wet, hipStream_t s) {
+  nsteps = n;
+  dh = want_dh;
+  wet = want_wet;
+  if (n < 1 || (!want_dh && !want_wet)) return hipSuccess;
+  const int64_t held = n < kSeriesChunk ? n : kSeriesChunk;
+  hipError_t e = hipMalloc((void**)&slots, sizeof(unsigned long long) * held * kSeriesSlots *
+                                               kSeriesWords);
+  if (e != hipSuccess) slots = nullptr;
+  if (e == hipSuccess) e = hipMalloc((void**)&folded, sizeof(double) * 3 * n);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_series_init, dim3(64), dim3(256), 0, s, slots, held);
+  return hipGetLastError();
+}
+
+void SeriesRun::taken(int64_t i, int64_t k, hipStream_t s) {
+  const int64_t end = i + k;
+  if (!slots || (end % kSeriesChunk != 0 && end != nsteps)) return;
+  const int64_t first = (end - 1) / kSeriesChunk * kSeriesChunk;
+  hipLaunchKernelGGL(k_series_fold, dim3((unsigned)(end - first)), dim3(64), 0, s, slots,
+                     folded + 3 * first);
+}
+
+hipError_t SeriesRun::fetch(double* out, hipStream_t s) const {
+  const hipError_t e =
+      hipMemcpyAsync(out, folded, sizeof(double) * 3 * nsteps, hipMemcpyDeviceToHost, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
 
 template void launch_step<double>(const StepIO<double>&, const StepParams&, StepSeries, uint64_t,

@@ -786,7 +786,7 @@ __global__ __launch_bounds__(64) void k_strip_f32(TileIO io, F32K K, TileRun R, 
   const int y0 = sg * seg;
   const int S = min(seg, R.Ly - y0);
   SeriesAcc acc{-__builtin_inf(), __builtin_inf(), 0u};
-  const bool series = ser.dh_keys || ser.wet;
+  const bool series = ser.base != nullptr;
   with_store_mode(R.nts, [&](auto mode) {
     constexpr int NTS = decltype(mode)::value;
     if (series) strip_run<READ_FT, THERMAL, true, NTS>(io, K, R, st * kStripOut, y0, S, acc);
@@ -802,11 +802,7 @@ __global__ __launch_bounds__(64) void k_strip_f32(TileIO io, F32K K, TileRun R, 
     lcnt += __shfl_xor(lcnt, o);
   }
   if ((threadIdx.x & 63) == 0) {
-    if (ser.dh_keys) {
-      atomicMax(&ser.dh_keys[0], kmax);
-      atomicMin(&ser.dh_keys[1], kmin);
-    }
-    if (ser.wet) atomicAdd(&ser.wet[0], (unsigned long long)lcnt);
+    ser.add(0, kmax, kmin, lcnt);
   }
 }
 
@@ -837,11 +833,7 @@ __device__ __forceinline__ void series_flush(const SeriesAcc& acc, const StepSer
       kmin = red_k[2 * w + 1] < kmin ? red_k[2 * w + 1] : kmin;
       lcnt += red_c[w];
     }
-    if (ser.dh_keys) {
-      atomicMax(&ser.dh_keys[0], kmax);
-      atomicMin(&ser.dh_keys[1], kmin);
-    }
-    if (ser.wet) atomicAdd(&ser.wet[0], (unsigned long long)lcnt);
+    ser.add(0, kmax, kmin, lcnt);
   }
 }
 
@@ -853,7 +845,7 @@ __device__ __forceinline__ void single_film_step(const TileIO& io, const F32K& K
   const int tile = tile_of_block(ntx, ntiles, R.step);
   const int x0 = (tile % ntx) * TXW, y0 = (tile / ntx) * TY;
   SeriesAcc acc{-__builtin_inf(), __builtin_inf(), 0u};
-  const bool series = ser.dh_keys || ser.wet;
+  const bool series = ser.base != nullptr;
   if (series) tile_step<TXW, NTH, TY, READ_FT, THERMAL, SRC, true>(io, K, R, x0, y0, sm, acc);
   else tile_step<TXW, NTH, TY, READ_FT, THERMAL, SRC, false>(io, K, R, x0, y0, sm, acc);
   if (series) series_flush<NW>(acc, ser, red_k, red_c);

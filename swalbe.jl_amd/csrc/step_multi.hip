@@ -138,7 +138,7 @@ struct Multi {
       }
       cnt += (unsigned int)__popcll(__ballot(own && hv > sp.wet_thresh));
     }
-    if (R.ser.dh_keys)
+    if (R.ser.dh)
       for (int o = 32; o > 0; o >>= 1) {
         const double a = __shfl_xor(mx, o), b = __shfl_xor(mn, o);
         mx = a > mx ? a : mx;
@@ -160,11 +160,7 @@ struct Multi {
       mn = red[3 * w + 1] < mn ? red[3 * w + 1] : mn;
       cnt += red[3 * w + 2];
     }
-    if (R.ser.dh_keys) {
-      atomicMax(&R.ser.dh_keys[2 * i], dkey(mx));
-      atomicMin(&R.ser.dh_keys[2 * i + 1], dkey(mn));
-    }
-    if (R.ser.wet && cnt > 0.0) atomicAdd(&R.ser.wet[i], (unsigned long long)cnt);
+    R.ser.add(i, dkey(mx), dkey(mn), (unsigned long long)cnt);
   }
 
   // film pressure (src/pressure.jl:119-155)
@@ -384,7 +380,7 @@ struct Multi {
       const int64_t i = S - (K - R.k);
       if (i >= 0) {
         constexpr bool LAST = S == K - 1;
-        const bool ser = R.ser.dh_keys || R.ser.wet;
+        const bool ser = R.ser.base != nullptr;
         if (ser) series(red);
         pressure<3 * S + 1>(LAST && R.write_f);
         __syncthreads();
