@@ -262,7 +262,7 @@ int swalbe_create(int32_t Lx, int32_t Ly, int32_t dtype, int32_t kind, swalbe_st
                    &F.hgpx,    &F.hgpy,     &F.kbtx,   &F.kbty};
   for (void** p : scal)
     if (rc == SWALBE_OK) rc = alloc_field(p, fb);
-  st->nparts = (int)std::min<int64_t>(kMaxParts, std::max<int64_t>(1, F.N / 4096));
+  st->nparts = (int)std::min<int64_t>(kMaxParts, std::max<int64_t>(1, F.N / 1024));
   if (rc == SWALBE_OK) rc = alloc_field((void**)&st->partials, sizeof(double) * 4 * kMaxParts);
   if (rc == SWALBE_OK) rc = alloc_field((void**)&st->red_out, sizeof(double) * 4);
   if (rc == SWALBE_OK) {

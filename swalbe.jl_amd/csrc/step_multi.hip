@@ -118,12 +118,15 @@ struct Multi {
       }
   }
 
-  // max, min and count(> thresh) of the step's input height over the tile's nodes, one result
-  // per wave in `red`
-  __device__ __forceinline__ void series(double* red) const {
+  // max, min and count(> thresh) of the step's input height over the tile's nodes, gathered by
+  // LDS atomics that nobody waits for before the next barrier (a shuffle tree per wave and one
+  // thread walking the waves' results took 1.2 us a step, half a step of a 100 x 100 film);
+  // eight addresses share the lanes of a wave
+  __device__ __forceinline__ void series(unsigned long long* red) const {
     using I = Inner<RW, RH, 3 * K, NT>;
-    double mx = -__builtin_inf(), mn = __builtin_inf();
+    unsigned long long kmax = 0ull, kmin = ~0ull;
     unsigned int cnt = 0;
+    bool any = false;
 #pragma unroll
     for (int q = 0; q < I::NQ; ++q) {
       const int o = I::off(q);
@@ -133,34 +136,39 @@ struct Multi {
       if (own) {
         hv = (double)plane(kH)[o];
         if constexpr (F32) hv = (double)K32.href + hv;
-        mx = hv > mx ? hv : mx;
-        mn = hv < mn ? hv : mn;
+        const unsigned long long key = dkey(hv);
+        kmax = key > kmax ? key : kmax;
+        kmin = key < kmin ? key : kmin;
+        any = true;
       }
       cnt += (unsigned int)__popcll(__ballot(own && hv > sp.wet_thresh));
     }
-    if (R.ser.dh)
-      for (int o = 32; o > 0; o >>= 1) {
-        const double a = __shfl_xor(mx, o), b = __shfl_xor(mn, o);
-        mx = a > mx ? a : mx;
-        mn = b < mn ? b : mn;
-      }
-    if ((threadIdx.x & 63) == 0) {
-      double* w = red + 3 * (threadIdx.x >> 6);
-      w[0] = mx;
-      w[1] = mn;
-      w[2] = (double)cnt;
+    if (R.ser.dh && any) {
+      atomicMax(&red[2 * (threadIdx.x & 7)], kmax);
+      atomicMin(&red[2 * (threadIdx.x & 7) + 1], kmin);
     }
+    if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(&red[16], (unsigned long long)cnt);
   }
 
-  __device__ __forceinline__ void series_out(const double* red, int64_t i) const {
+  // after the barrier: the tile's result to the step's slot, the LDS words neutral again (the
+  // next step's series comes after two more barriers)
+  __device__ __forceinline__ void series_out(unsigned long long* red, int64_t i) const {
     if (threadIdx.x != 0) return;
-    double mx = red[0], mn = red[1], cnt = red[2];
-    for (int w = 1; w < NT / 64; ++w) {
-      mx = red[3 * w] > mx ? red[3 * w] : mx;
-      mn = red[3 * w + 1] < mn ? red[3 * w + 1] : mn;
-      cnt += red[3 * w + 2];
+    unsigned long long kmax = 0ull, kmin = ~0ull;
+    if (R.ser.dh)
+      for (int w = 0; w < 8; ++w) {
+        kmax = red[2 * w] > kmax ? red[2 * w] : kmax;
+        kmin = red[2 * w + 1] < kmin ? red[2 * w + 1] : kmin;
+      }
+    R.ser.add(i, kmax, kmin, red[16]);
+    series_clear(red);
+  }
+  static __device__ __forceinline__ void series_clear(unsigned long long* red) {
+    for (int w = 0; w < 8; ++w) {
+      red[2 * w] = 0ull;
+      red[2 * w + 1] = ~0ull;
     }
-    R.ser.add(i, dkey(mx), dkey(mn), (unsigned long long)cnt);
+    red[16] = 0ull;
   }
 
   // film pressure (src/pressure.jl:119-155)
@@ -375,7 +383,7 @@ struct Multi {
 
   // step S of K (those before K - R.k are not taken), then the ones after it
   template <int S>
-  __device__ __forceinline__ void steps(double* red) const {
+  __device__ __forceinline__ void steps(unsigned long long* red) const {
     if constexpr (S < K) {
       const int64_t i = S - (K - R.k);
       if (i >= 0) {
@@ -399,9 +407,10 @@ template <typename T, int TX, int TY, int K, int NT, bool RFT, bool TH, bool GRA
 __global__ __launch_bounds__(NT) void k_multi(StepIO<T> io, StepParams sp, F32K K32, MultiRun R) {
   using M = Multi<T, TX, TY, K, NT, RFT, TH, GRAV>;
   __shared__ T lds[kPlanes * M::RN];
-  __shared__ double red[3 * (NT / 64)];
+  __shared__ unsigned long long red[17];
   const int tile = blockIdx.x;
   const M m{io, sp, K32, R, lds, (tile % R.ntx) * TX, (tile / R.ntx) * TY};
+  if (threadIdx.x == 0) M::series_clear(red);
   m.load(3 * (K - R.k));
   __syncthreads();
   m.template steps<0>(red);

@@ -1,5 +1,5 @@
 """Reductions over several workgroups and their finishing wave, at the sizes
-where the number of partials changes (2D: one per 4096 nodes, at most 1024,
+where the number of partials changes (2D: one per 1024 nodes, at most 1024,
 64 lanes; 1D: one per 4096 nodes, at most 256).  max, min and count are exact;
 the sum of n positive terms in any tree order is within (log2 n + 64) ulp of
 the exact sum (a lane adds at most 64 terms in a row here per 4096 nodes)."""
