@@ -23,7 +23,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIBDIR = os.path.join(PKG, "lib")
 OBJDIR = os.path.join(PKG, "_build")
 LIB = os.path.join(LIBDIR, "libswalbe_hip.so")
-SOURCES = ["api.hip", "ops.hip", "step.hip", "step_f32.hip", "step_multi.hip", "batch.hip", "serve.hip",
+SOURCES = ["api.hip", "ops.hip", "step.hip", "step_f32.hip", "step_multi.hip", "step_march.hip", "batch.hip", "serve.hip",
            "d1q3.hip", "measure.hip", "xfer.hip"]
 PROBE_SOURCES = ["probe.hip"]
 PROBE_LIB = os.path.join(LIBDIR, "libswalbe_probe.so")

@@ -812,7 +812,7 @@ struct LoopBuffers {
 // `multi`: nsub steps from t in one launch of its shape (geom >= 0).
 template <typename T>
 void enqueue_step(swalbe_state* st, const StepParams& sp, StepSeries ser, uint64_t t, int tile_y,
-                  int variant, int nts, bool outs, const MultiShape& multi, int nsub) {
+                  int variant, int nts, bool outs, const MultiShape& multi, int nsub, int march) {
   Film& F = st->film;
   const int cur = F.hu_cur;
   const int fdst = F.fout_buf != F.ftemp_buf ? F.fout_buf : 1 - F.ftemp_buf;
@@ -830,6 +830,12 @@ void enqueue_step(swalbe_state* st, const StepParams& sp, StepSeries ser, uint64
   if (multi.geom >= 0) {
     launch_multi<T>(io, sp, ser, t, nsub, outs, F.Lx, F.Ly, F.fstride, F.enc, multi.geom,
                     st->stream);
+    F.fout_buf = F.ftemp_buf = fdst;
+    F.hu_cur = 1 - cur;
+    return;
+  }
+  if (march > 0) {
+    launch_march<T>(io, sp, ser, t, outs, F.Lx, F.Ly, F.fstride, F.enc, march, st->stream);
     F.fout_buf = F.ftemp_buf = fdst;
     F.hu_cur = 1 - cur;
     return;
@@ -992,6 +998,9 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
   const bool automatic = o->variant == 0 && o->tile_y <= 0;
   const MultiShape multi = automatic ? multi_shape(F.Lx, F.Ly, F.dtype == SWALBE_F64)
                                      : MultiShape{-1, 1};
+  // large films whose loop writes f and p on its last step only march in strips
+  const int march =
+      automatic && multi.geom < 0 && final_only ? march_segment(F.Lx, F.Ly) : 0;
   auto steps_at = [&](int64_t it) -> int64_t {
     if (multi.geom < 0 || want_meas) return 1;
     int64_t k = std::min<int64_t>(multi.k, nsteps - it);
@@ -1023,10 +1032,10 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
     const bool outs = multi.geom >= 0 ? it == nsteps : !final_only || it == nsteps;
     if (F.dtype == SWALBE_F64)
       enqueue_step<double>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
-                           multi, (int)nsub);
+                           multi, (int)nsub, march);
     else
       enqueue_step<float>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
-                           multi, (int)nsub);
+                           multi, (int)nsub, march);
     series.taken(it - 1, nsub, st->stream);
     if (want_snap && (t + nsub - 1) % o->snap_every == 0) {
       const int r = (int)(ksnap % SnapRing::R);

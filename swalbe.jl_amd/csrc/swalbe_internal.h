@@ -260,6 +260,14 @@ void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int geom,
                   hipStream_t s);
 
+// One τ = 1 step of a large film, a wave per strip of columns and segment of
+// `seg` rows (step_march.hip), writing the moments, and f and p with write_f.
+// march_segment: the rows per segment for a film, 0 where tiles are faster.
+int march_segment(int Lx, int Ly);
+template <typename T>
+void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step,
+                  bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int seg, hipStream_t s);
+
 // Deterministic FP64 reductions of a field: sum, max, min, count(> thresh).
 template <typename T>
 void launch_reduce(const T* h, int64_t N, double href, double thresh, double* partials,
