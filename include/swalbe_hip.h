@@ -193,7 +193,9 @@ typedef struct swalbe_step_opts {
     int32_t surf_theta_field; /* reduced energy from the θ field (else cos πθ of params) */
     /* 1: with τ = 1, write the distributions and the pressure on the last
      * step only (no step reads them, so every result is the same); the
-     * other fields are written every step.  Ignored when τ ≠ 1. */
+     * other fields are written every step.  Ignored when τ ≠ 1.  With
+     * variant = 0 and tile_y = 0 large films then run a kernel of their own:
+     * the same FP64 bits, FP32 to rounding. */
     int32_t final_outputs_only;
 } swalbe_step_opts;
 int swalbe_time_loop(swalbe_state *st, const swalbe_params *p, int64_t nsteps,

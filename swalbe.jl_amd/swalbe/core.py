@@ -618,9 +618,11 @@ def time_loop(sys: SysConst, state: HipState, *args, verbose: bool = False, ther
     surfacearea!'s area and reduced energy and fluid_dry!'s mask of every
     step's input height, taken on the device without host synchronisation
     (threshold measure_thresh; energy from the θ field with
-    surface_theta_field).  final_outputs_only (τ = 1) writes the
-    distributions and the pressure on the last step only: the same results
-    with 28 instead of 64 bytes per node and step in FP32.  A 1D state runs
+    surface_theta_field).  With τ = 1 no step reads the distributions or the
+    pressure of the one before, and nothing hands them out between steps, so
+    the loop writes them on its last step: 24 instead of 64 bytes per node and
+    step in FP32.  final_outputs_only asks for that also where tile_y or
+    variant name a kernel; without it those write every step's.  A 1D state runs
     the 1D loop (its own keywords:
     variant, γ, grad_gamma_sign, snapshots + dumping).  nontemporal
     sets the stores' cache policy (0, 1, 2: the same bits); by default
@@ -637,6 +639,7 @@ def time_loop(sys: SysConst, state: HipState, *args, verbose: bool = False, ther
     o = _lib.StepOpts()
     o.thermal, o.seed, o.t0, o.materialize, o.tile_y = int(thermal), int(seed), int(state.t), int(materialize), tile_y
     o.variant = int(variant)  # FP32 kernel: 0 default, 1 / 2 LDS tiles, 3 strips
+    final_outputs_only = P.τ == 1.0 and (bool(final_outputs_only) or (tile_y == 0 and variant == 0))
     o.nontemporal = int(nontemporal) if nontemporal is not None else store_mode(
         sys.Lx, sys.Ly, state.T is np.float64, final_outputs_only)
     keep = []
