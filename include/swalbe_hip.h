@@ -137,6 +137,14 @@ int swalbe_inclination(swalbe_state *st, double ax, double ay, double fac);
 /* state.Fx .= -state.h∇px .- state.slipx [.- state.kbtx]
  * -- src/simulate.jl:18-19, scripts/Rivulet_stability.jl:123-124 */
 int swalbe_force_sum(swalbe_state *st, int32_t with_thermal);
+/* One step of the op-by-op loop in two calls, for a callback between them
+ * (time_loop(sys, state, f, measure), src/simulate.jl:69-96): filmpressure!
+ * (scalar θ), h∇p!, slippage!, [thermal! of (seed, step)] and the force sum;
+ * then equilibrium!, BGKandStream! and moments!.  Every field those ops write
+ * is written, with the same bits. */
+int swalbe_step_forces(swalbe_state *st, const swalbe_params *p, int32_t thermal, uint64_t seed,
+                       uint64_t step);
+int swalbe_step_advance(swalbe_state *st, double g, double tau);
 
 /* ---- fused time loop: time_loop(sys, state[, θ | Δh | f, measure])
  * -- src/simulate.jl:6-96.  One kernel per step (collide + pull-stream +

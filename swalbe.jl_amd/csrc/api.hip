@@ -636,6 +636,29 @@ int swalbe_force_sum(swalbe_state* st, int32_t with_thermal) {
   return SWALBE_OK;
 }
 
+// One step's force half and its second half, for a loop with a callback
+// between them (src/simulate.jl:84-92).
+extern "C" int swalbe_step_forces(swalbe_state* st, const swalbe_params* p, int32_t thermal,
+                                  uint64_t seed, uint64_t step) {
+  SW_CHECK_STATE(st);
+  if (!p || p->n < 0 || p->m < 0) {
+    set_error("swalbe_step_forces: null params or negative exponent");
+    return SWALBE_EINVAL;
+  }
+  if (int rc = set_device(st)) return rc;
+  SW_BOTH(st, launch_forces<T>(st->film, *p, thermal ? 1 : 0, seed, step, st->stream));
+  SW_HIP(hipGetLastError());
+  return SWALBE_OK;
+}
+
+extern "C" int swalbe_step_advance(swalbe_state* st, double g, double tau) {
+  SW_CHECK_STATE(st);
+  if (int rc = set_device(st)) return rc;
+  SW_BOTH(st, launch_advance<T>(st->film, g, tau, st->stream));
+  SW_HIP(hipGetLastError());
+  return SWALBE_OK;
+}
+
 // ---------------------------------------------------------------- reductions
 static int reduce_enqueue(swalbe_state* st, const void* p, double href, double thresh,
                           double* out_dev) {
@@ -660,9 +683,13 @@ int swalbe_reduce(swalbe_state* st, int32_t field, double thresh, double out[4])
     set_error("swalbe_reduce: field not allocated");
     return SWALBE_EINVAL;
   }
-  if (int rc = reduce_enqueue(st, p, enc_offset(st->film, field, 0), thresh, st->red_out)) return rc;
-  SW_HIP(hipMemcpyAsync(out, st->red_out, 4 * sizeof(double), hipMemcpyDeviceToHost, st->stream));
-  SW_HIP(hipStreamSynchronize(st->stream));
+  HostResult res(st->device, st->stream);
+  // four doubles straight into pinned memory; without any, through the device
+  double* dst = res.dev() ? res.dev() : st->red_out;
+  if (int rc = reduce_enqueue(st, p, enc_offset(st->film, field, 0), thresh, dst)) return rc;
+  if (!res.dev())
+    SW_HIP(hipMemcpyAsync(out, dst, 4 * sizeof(double), hipMemcpyDeviceToHost, st->stream));
+  SW_HIP(res.get(out, 4));
   return SWALBE_OK;
 }
 

@@ -160,6 +160,15 @@ template <typename T>
 void launch_kappa_field(T* kap, const T* theta, int n, int m, double hmin, int64_t N,
                         hipStream_t s);
 
+// The two halves of an op-by-op step around a user's callback: filmpressure!,
+// h∇p!, slippage!, [thermal!] and the force sum; equilibrium!, BGKandStream!
+// and moments! (the moments change buffers).
+template <typename T>
+void launch_forces(const Film& F, const swalbe_params& p, int thermal, uint64_t seed, uint64_t step,
+                   hipStream_t s);
+template <typename T>
+void launch_advance(Film& F, double g, double tau, hipStream_t s);
+
 // ---------------------------------------------------------------- fused step
 struct StepParams {
   double gamma, kappa, hmin, hcrit;
@@ -296,6 +305,22 @@ int field_from_host(void* dev, size_t des, const void* host, size_t hes, int64_t
 // FP32 planes re-encoded in place from one set of offsets to another.
 void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const double* from,
                      const double* to, hipStream_t s);
+// A few doubles that a kernel writes straight into pinned host memory: pass
+// dev() to the kernel, then get() waits for the stream and copies them out.
+// dev() is null where no pinned memory is to be had.
+class HostResult {
+ public:
+  HostResult(int device, hipStream_t s);
+  ~HostResult();
+  double* dev() const { return p_; }
+  hipError_t get(double* out, int n);
+
+ private:
+  int device_;
+  hipStream_t s_;
+  void* stage_ = nullptr;
+  double* p_ = nullptr;
+};
 // Called once per film or batch at creation and destruction: the pinned
 // transfer buffers are kept while any exists.
 void xfer_retain();

@@ -23,12 +23,14 @@ namespace swalbe {
 
 namespace {
 
-constexpr size_t kChunk = (size_t)1 << 20;  // bytes of one pinned buffer
+constexpr size_t kChunk = (size_t)1 << 19;  // bytes of one pinned buffer
 constexpr size_t kKeep = 10;                // idle buffers kept per device while films live
-// threads that copy a field of this many bytes: 1, 2 from 2 MB, 4 from 8 MB
-// (67 MB into fresh memory: 5.2 ms with one, 1.8 with four, 1.9 with eight)
+// threads that copy a field of this many bytes: 1, 2 from 4 MB, 4 from 8 MB
+// (67 MB into fresh memory: 5.2 ms with one, 1.8 with four, 1.9 with eight;
+// a first upload of 2 MB, with its buffers to be allocated, takes 260 us with
+// two threads and buffers of 1 MB, 190 with one and 512 KB)
 inline int copy_threads(size_t bytes) {
-  return bytes >= ((size_t)8 << 20) ? 4 : bytes >= ((size_t)2 << 20) ? 2 : 1;
+  return bytes >= ((size_t)8 << 20) ? 4 : bytes >= ((size_t)4 << 20) ? 2 : 1;
 }
 
 // ---------------------------------------------------------------- pinned buffers
@@ -296,6 +298,27 @@ void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const do
   const int64_t b = (n + 255) / 256;
   hipLaunchKernelGGL(k_reencode, dim3((unsigned)(b < 65535 ? b : 65535), (unsigned)planes),
                      dim3(256), 0, s, dev, n, stride, offsets(from, planes), offsets(to, planes));
+}
+
+HostResult::HostResult(int device, hipStream_t s) : device_(device), s_(s) {
+  Stage* st = new Stage;
+  if (stage_take(device, st) != hipSuccess) (void)hipGetLastError();
+  stage_ = st;
+  p_ = (double*)st->pin;
+}
+
+HostResult::~HostResult() {
+  Stage* st = (Stage*)stage_;
+  // whatever was launched may still write: the buffer goes back when it cannot
+  if (st->pin) (void)hipStreamSynchronize(s_);
+  stage_give(*st);
+  delete st;
+}
+
+hipError_t HostResult::get(double* out, int n) {
+  const hipError_t e = hipStreamSynchronize(s_);
+  if (e == hipSuccess && p_) memcpy(out, p_, sizeof(double) * (size_t)n);
+  return e;
 }
 
 void xfer_retain() {

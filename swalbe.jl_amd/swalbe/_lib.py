@@ -140,6 +140,8 @@ def lib():
     _sig(L, "swalbe_thermal", [_V, _D, _D, _D, C.c_uint64, C.c_uint64])
     _sig(L, "swalbe_inclination", [_V, _D, _D, _D])
     _sig(L, "swalbe_force_sum", [_V, _I])
+    _sig(L, "swalbe_step_forces", [_V, C.POINTER(Params), _I, C.c_uint64, C.c_uint64])
+    _sig(L, "swalbe_step_advance", [_V, _D, _D])
     _sig(L, "swalbe_time_loop", [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts)])
     _sig(L, "swalbe_time_loop_timed",
          [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts), C.POINTER(_D)])

@@ -719,21 +719,27 @@ def time_loop(sys: SysConst, state: HipState, *args, verbose: bool = False, ther
 
 
 def _time_loop_callback(sys, state, f: Callable, measure, verbose, thermal, seed):
-    """Per-op loop for an arbitrary measurement callback (src/simulate.jl:69-96)."""
+    """Op-by-op loop for an arbitrary measurement callback
+    (src/simulate.jl:69-96): the ops before f in one call, those after it in
+    another, every field of the state written as the single ops would.  f may
+    change the state and sys.param."""
     P = sys.param
+    L = lib()
     for _ in range(P.Tmax):
         t = state.t + 1
         if P.tdump > 0 and t % P.tdump == 0 and verbose:
             print(f"Time step {t} mass is {round(state.reduce()['sum'], 3)}")
-        filmpressure(state, sys)
-        h_grad_p(state)
-        slippage(state, sys)
-        if thermal:
-            check(lib().swalbe_thermal(state.handle, P.kbt, P.μ, P.δ, int(seed), int(t)), "thermal")
-        force_sum(state, thermal)
+        if np.ndim(P.θ) == 0:
+            check(L.swalbe_step_forces(state.handle, C.byref(P.cparams()), int(bool(thermal)),
+                                       int(seed), int(t)), "step_forces")
+        else:  # f made θ a field
+            filmpressure(state, sys)
+            h_grad_p(state)
+            slippage(state, sys)
+            if thermal:
+                check(L.swalbe_thermal(state.handle, P.kbt, P.μ, P.δ, int(seed), int(t)), "thermal")
+            force_sum(state, thermal)
         f(measure, state)
-        equilibrium(state, sys)
-        BGKandStream(state, sys)
-        moments(state)
+        check(L.swalbe_step_advance(state.handle, float(P.g), float(P.τ)), "step_advance")
         state.t = t
     return state, measure
