@@ -118,7 +118,8 @@ def batch_run(steps, warmup, graph_steps=100, autotune=True, final_outputs_only=
     """256 independent droplet-coalescence films (Lx in {128..1024} step 64,
     Ly = Lx/2, two tangent caps, per-film θ, γ, radius) stepped together by
     the batched FP32 kernel; `steps` timed batch steps after `warmup`, run as
-    captured graphs.  Each film's tile height (8 or 16 rows) is the one the
+    captured graphs (distributions and pressure are written by each graph's
+    last step).  Each film's tile height (8 or 16 rows) is the one the
     autotuner measured fastest for its shape (the tuning runs at admission,
     before the timed steps, and is reported).  nontemporal >= 0 sets the
     films' store mode (otherwise the batch's default, 2)."""
@@ -158,7 +159,8 @@ def bench_batch(a):
     """Config 4 on its own line (coalesce256_batch): see batch_run()."""
     r = batch_run(a.steps, a.warmup, a.graph_steps, not a.no_autotune,
                   nontemporal=a.nontemporal)
-    bpl = bytes_per_lup(4, True)
+    # h, ux, uy in and out each step; the populations and p once per graph
+    bpl = 24 + 40 / max(1, a.graph_steps or a.steps)
     achieved = bpl * r["glups"]
     line = {
         "metric": "GLUPS of 256 batched FP32 droplet-coalescence films (one launch per step)",
@@ -173,7 +175,7 @@ def bench_batch(a):
                    "parallelism": "single GPU", "finite": r["finite"]},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": None, "bytes_per_lup": bpl},
+                     "traffic": None, "bytes_per_lup": round(bpl, 2)},
         "autotune": {"on": not a.no_autotune, "shapes": len(r["shapes"]),
                      "films_rows8": r["rows"].count(8), "films_rows16": r["rows"].count(16),
                      "rows_by_shape": r["shapes"], "admission_s": round(r["admit_s"], 3)},
@@ -758,8 +760,8 @@ def main():
                                   "both ways, wall clock)"},
     }
     if not a.no_batch and (Lx, Ly, dt) == (4096, 4096, "f32"):
-        # config 4: 256 films in one launch per step, every step's outputs
-        # written (its own line: --workload coalesce256_batch)
+        # config 4: 256 films in one launch per step
+        # (its own line: --workload coalesce256_batch)
         r = batch_run(300, 20)
         line["batch"] = {"workload": BATCH_DESC, "GLUPS": round(r["glups"], 3),
                          "ms_per_step": round(r["ms"] / 300, 5), "steps": 300, "warmup": 20,

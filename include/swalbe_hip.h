@@ -298,9 +298,11 @@ int swalbe_batch_tune_shape(const swalbe_params *p, int32_t Lx, int32_t Ly,
                             double *ms_rows16);
 /* tile height (8 or 16) of a resident film */
 int swalbe_batch_film_tile_y(swalbe_batch *b, int32_t slot, int32_t *tile_y);
-/* Films admitted after this call with τ = 1 write their distributions and
- * pressure on their last step only (their heights and velocities every
- * step): the same final state for less traffic.  Downloading FOUT or
+/* A film with τ = 1 writes its distributions and pressure on the last step of
+ * each swalbe_batch_step call (or captured graph); its heights and velocities
+ * every step.  Films admitted after this call with τ = 1 write them on their
+ * own last step only: the same final state for less traffic still where a run
+ * is cut into short calls.  Downloading FOUT or
  * PRESSURE of such a film before it finishes is an error.  The native
  * server sets it (its requests return heights). */
 int swalbe_batch_set_final_outputs_only(swalbe_batch *b, int32_t on);

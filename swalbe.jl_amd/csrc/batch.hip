@@ -262,9 +262,8 @@ int enqueue_steps(swalbe_batch* b, int64_t nsteps) {
     }
     if (!b->gexec) {
       SW_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeGlobal));
-      for (int i = 0; i < b->graph_steps; ++i)
-        launch_batch_f32(b->films(), b->tstart(), b->hdr(), b->d_counter, grid, b->nts, any,
-                         b->stream);
+      launch_batch_f32(b->films(), b->tstart(), b->hdr(), b->d_counter, grid, b->graph_steps,
+                       b->nts, any, b->stream);
       hipError_t e = hipStreamEndCapture(b->stream, &b->graph);
       if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
       SW_HIP(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
@@ -275,9 +274,12 @@ int enqueue_steps(swalbe_batch* b, int64_t nsteps) {
       done += b->graph_steps;
     }
   }
-  for (; done < nsteps; ++done)
-    launch_batch_f32(b->films(), b->tstart(), b->hdr(), b->d_counter, grid, b->nts, any,
+  while (done < nsteps) {
+    const int k = (int)std::min<int64_t>(nsteps - done, 1 << 30);
+    launch_batch_f32(b->films(), b->tstart(), b->hdr(), b->d_counter, grid, k, b->nts, any,
                      b->stream);
+    done += k;
+  }
   SW_HIP(hipGetLastError());
   b->counter += (unsigned long long)nsteps;
   return record_steps_event(b);
@@ -616,13 +618,14 @@ int swalbe_batch_add(swalbe_batch* b, const swalbe_params* p, int32_t Lx, int32_
   // initial state: h from the spec, u = 0, p = 0, f_t = feq(h, 0) when τ ≠ 1
   // heights are stored relative to the FP32 reference height the kernel adds
   launch_film_init<float>(d.h[0], Lx, Ly, *init, (double)s.enc.href, b->stream);
-  for (int i = 2; i < 7; ++i) launch_fill<float>(q[i], 0.0, (int64_t)N, b->stream);
-  if (two_f)
+  // q[2] .. q[6] and the distributions lie one behind the other: one fill
+  const size_t zeroed = two_f ? 5 : 5 + kQ;
+  launch_fill<float>(q[2], 0.0, (int64_t)(zeroed * (plane / 4)), b->stream);
+  if (two_f) {
     launch_equilibrium<float>(d.f[0], d.h[0], d.ux[0], d.uy[0], d.p, p->g, Lx, Ly, d.fstride,
                               s.enc, b->stream);
-  else
-    launch_fill<float>(d.f[0], 0.0, (int64_t)9 * d.fstride, b->stream);
-  launch_fill<float>(d.p, 0.0, (int64_t)N, b->stream);
+    launch_fill<float>(d.p, 0.0, (int64_t)N, b->stream);
+  }
   SW_HIP(hipGetLastError());
   b->dirty = true;
   *slot_out = slot;

@@ -59,11 +59,12 @@ struct BatchHdr {
   int total_tiles;
 };
 
-// One batched step (all resident films) followed by the counter increment.
+// `steps` >= 1 batched steps (all resident films), then the counter's increment.
+// Films with τ = 1 write f and p on the last of them (and on their own last).
 // any_ft: some resident film has τ ≠ 1 (reads f_t); the kernel without that
 // path needs fewer registers and holds one more workgroup per CU.
 void launch_batch_f32(const BatchFilm* films, const int* tstart, const BatchHdr* hdr,
-                      unsigned long long* counter, int grid, int nts, bool any_ft,
+                      unsigned long long* counter, int grid, int steps, int nts, bool any_ft,
                       hipStream_t s);
 int batch_blocks_per_cu(bool any_ft);
 
