@@ -176,6 +176,7 @@ struct Job {
   int planes, device;
   Offsets off;
   bool bits;
+  bool single;  // one chunk: its end is the stream's, no event (0.9 us less of 16)
   hipStream_t s;
   std::atomic<int64_t> next{0};
   std::atomic<int> err{0};
@@ -206,7 +207,7 @@ hipError_t issue(const Job& J, Stage& st, int64_t a, int64_t b) {
     else launch_piece<float, float, false>(J, st.pin, P, grid);
   }
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipEventRecord(st.ev, J.s);
+  if (e == hipSuccess && !J.single) e = hipEventRecord(st.ev, J.s);
   return e;
 }
 
@@ -219,7 +220,7 @@ void run_chunks(Job* pJ) {
   hipError_t e = hipSetDevice(J.device);
   auto finish = [&](int r) {  // wait for buffer r; a download's chunk goes to the caller
     if (b[r] < 0) return;
-    const hipError_t w = hipEventSynchronize(st[r].ev);
+    const hipError_t w = J.single ? hipStreamSynchronize(J.s) : hipEventSynchronize(st[r].ev);
     if (w == hipSuccess && J.down && e == hipSuccess)
       memcpy(J.host + (size_t)a[r] * J.hes, st[r].pin, (size_t)(b[r] - a[r]) * J.hes);
     if (e == hipSuccess) e = w;
@@ -262,6 +263,7 @@ int transfer(bool down, void* host, size_t hes, void* dev, size_t des, int64_t n
   J.planes = planes;
   J.total = n * planes;
   J.per = (int64_t)(kChunk / hes);
+  J.single = J.total <= J.per;
   J.device = device;
   J.off = offsets(off, planes);
   J.bits = hes == des;
