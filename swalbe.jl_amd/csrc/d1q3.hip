@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "step_node.h"
 #include "swalbe_internal.h"
 
 using swalbe::dkey;
@@ -433,6 +434,10 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step, swalbe::St
   }
 }
 
+// a / d, correctly rounded
+__device__ __forceinline__ double quotient(double a, double d) { return swalbe::Recip(d).div(a); }
+__device__ __forceinline__ float quotient(float a, float d) { return a / d; }
+
 // Pointers read from the film table are generic to the compiler, which then
 // emits flat loads and stores (they wait on the LDS counter as well).  All of
 // them address global memory: say so.
@@ -476,14 +481,18 @@ __device__ __forceinline__ T from_above(T v) {
 // launch reads); the loop's last step runs in k1_step, which writes every
 // output.
 //
-// What bounds it: FP64 issue (about 100 instructions per node and step, three
-// IEEE divisions among them).  One node per lane takes 0.28 us a step however
-// short the film; the 2.2 us of a launch are shared by its k steps.  Measured
-// against the kernels it replaces for single films (us per step): L = 1024
-// 4.6 in one workgroup's LDS -> 0.51, over up to 256 CUs instead of one;
-// L = 3e6 36.4 with one launch and 64 bytes per node and step -> 12.2, with
-// 6 bytes per node and step.
-// EXTRA: any of the κ, γ, ∇γ fields or walls; RFT: τ ≠ 1; TH: noise.
+// What bounds it: FP64 issue (about 85 instructions per node and step, three
+// correctly rounded divisions among them).  One node per lane takes 0.25 us a
+// step however short the film; the 2.2 us of a launch are shared by its k
+// steps.  Measured against the kernels it replaces for single films (us per
+// step): L = 1024 4.6 in one workgroup's LDS -> 0.45, over up to 256 CUs
+// instead of one; L = 3e6 36.4 with one launch and 64 bytes per node and step
+// -> 10.0, with 6 bytes per node and step.
+// The loop exists twice: for the usual law, n = 9, m = 3 and g = 0, without a
+// branch per node, so that the division chains of a lane's nodes overlap, and
+// for any other (one copy with the branches and the compiler's division: 0.51
+// us at L = 1024, 12.2 at 3e6).
+// EXTRA: any of the κ, γ, ∇γ fields, walls or a body force; RFT: τ ≠ 1; TH: noise.
 template <typename T, int NPT, bool RFT, bool TH, bool EXTRA>
 __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, int W,
                                               swalbe::StepSeries ser) {
@@ -529,104 +538,116 @@ __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, in
   const T c6mu = (T)S.c6mu, c6d = (T)S.c6d, c3dd = (T)S.c3dd;
   const T omeg = (T)S.omeg, itau = (T)S.itau;
   const int own0 = 3 * k - lane * NPT;  // nodes j with own0 <= j < own0 + W are this wave's
+  auto run = [&](auto sel) {
+    constexpr bool usual = decltype(sel)::value;
 #pragma unroll 1
-  for (int s = 0; s < k; ++s) {
-    if (ser.base) {  // series over the step's input height
-      unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
+    for (int s = 0; s < k; ++s) {
+      if (ser.base) {  // series over the step's input height
+        unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
 #pragma unroll
-      for (int j = 0; j < NPT; ++j)
-        if (j >= own0 && j < own0 + W && xs + j < L) {
-          const double hv = (double)h[j];
-          const unsigned long long q = dkey(hv);
-          kmax = q > kmax ? q : kmax;
-          kmin = q < kmin ? q : kmin;
-          cnt += hv > S.wet_thresh ? 1ull : 0ull;
-        }
-      for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
-        kmax = a > kmax ? a : kmax;
-        kmin = b < kmin ? b : kmin;
-        cnt += __shfl_xor(cnt, o);
-      }
-      if (lane == 0) ser.add(s, kmax, kmin, cnt);
-    }
-    T p[NPT];
-    {
-      const T hl = from_below(h[NPT - 1]), hr = from_above(h[0]);
-#pragma unroll
-      for (int j = 0; j < NPT; ++j) {
-        const T hm = j > 0 ? h[j > 0 ? j - 1 : 0] : hl;
-        const T hp = j < NPT - 1 ? h[j < NPT - 1 ? j + 1 : 0] : hr;
-        const T a = hmin / (h[j] + hcrit);
-        const T v = -gam[j] * (kap[j] * disjoin_law(a, n, m));
-        p[j] = v - gam[j] * ((hm - T(2) * h[j]) + hp);
-      }
-    }
-    // forces and the collision at the source: f0 -> h, f1 -> u, f2 apart
-    T f2[NPT];
-    {
-      const T pl = from_below(p[NPT - 1]), pr = from_above(p[0]);
-#pragma unroll
-      for (int j = 0; j < NPT; ++j) {
-        const T pm = j > 0 ? p[j > 0 ? j - 1 : 0] : pl;
-        const T pp = j < NPT - 1 ? p[j < NPT - 1 ? j + 1 : 0] : pr;
-        const T hh = h[j];
-        const T hgp = (hh * T(-0.5)) * (pm - pp);
-        T F = -hgp - slip_node(hh, u[j], c6mu, c6d, c3dd);
-        if constexpr (TH)
-          F = F - noise_node<T>(S.seed, step0 + (uint64_t)s, xw[j]) *
-                      noise_amp(hh, (T)S.kb26, (T)S.delta);
-        if constexpr (EXTRA) {
-          if (S.gg) F = S.gg_sign < 0 ? F - gg[j] : F + gg[j];
-        }
-        if (S.body) F = F + (hh * (T)S.alpha) * (T)S.fac;
-        T e0, e1, e2;
-        feq_node(hh, u[j], g, e0, e1, e2);
-        if constexpr (RFT) {
-          h[j] = omeg * t0[j] + itau * e0;
-          u[j] = (omeg * t1[j] + itau * e1) + T(0.5) * F;
-          f2[j] = (omeg * t2[j] + itau * e2) - T(0.5) * F;
-        } else {  // τ = 1: 1/τ = 1 and no f_t
-          h[j] = e0;
-          u[j] = e1 + T(0.5) * F;
-          f2[j] = e2 - T(0.5) * F;
-        }
-      }
-    }
-    // pull-stream (bounce-back at walls) and moments
-    {
-      const T fl = from_below(u[NPT - 1]), fr = from_above(f2[0]);
-      T bl = T(0), br = T(0);
-      if constexpr (EXTRA) {
-        bl = from_below(b1[NPT - 1]);
-        br = from_above(b2[0]);
-      }
-      T prev1 = fl, prevb = bl;  // f1 and b1 of the node before
-#pragma unroll
-      for (int j = 0; j < NPT; ++j) {
-        const T s1 = u[j], s2 = f2[j];
-        const T f0 = h[j];
-        T f1 = prev1, fb = j < NPT - 1 ? f2[j < NPT - 1 ? j + 1 : 0] : fr;
-        if constexpr (EXTRA) {
-          if (walls) {
-            const T bp = j < NPT - 1 ? b2[j < NPT - 1 ? j + 1 : 0] : br;
-            f1 = (f1 - f1 * prevb) + s2 * b2[j];
-            fb = (fb - fb * bp) + s1 * b1[j];
+        for (int j = 0; j < NPT; ++j)
+          if (j >= own0 && j < own0 + W && xs + j < L) {
+            const double hv = (double)h[j];
+            const unsigned long long q = dkey(hv);
+            kmax = q > kmax ? q : kmax;
+            kmin = q < kmin ? q : kmin;
+            cnt += hv > S.wet_thresh ? 1ull : 0ull;
           }
-          prevb = b1[j];
+        for (int o = 32; o > 0; o >>= 1) {
+          const unsigned long long a = __shfl_xor(kmax, o), b = __shfl_xor(kmin, o);
+          kmax = a > kmax ? a : kmax;
+          kmin = b < kmin ? b : kmin;
+          cnt += __shfl_xor(cnt, o);
         }
-        prev1 = s1;
-        if constexpr (RFT) {
-          t0[j] = f0;
-          t1[j] = f1;
-          t2[j] = fb;
+        if (lane == 0) ser.add(s, kmax, kmin, cnt);
+      }
+      T p[NPT];
+      {
+        const T hl = from_below(h[NPT - 1]), hr = from_above(h[0]);
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) {
+          const T hm = j > 0 ? h[j > 0 ? j - 1 : 0] : hl;
+          const T hp = j < NPT - 1 ? h[j < NPT - 1 ? j + 1 : 0] : hr;
+          const T a = quotient(hmin, h[j] + hcrit);
+          const T v = -gam[j] * (kap[j] * disjoin_law(a, usual ? 9 : n, usual ? 3 : m));
+          p[j] = v - gam[j] * ((hm - T(2) * h[j]) + hp);
         }
-        const T hn = (f0 + f1) + fb;
-        h[j] = hn;
-        u[j] = (f1 - fb) / hn;
+      }
+      // forces and the collision at the source: f0 -> h, f1 -> u, f2 apart
+      T f2[NPT];
+      {
+        const T pl = from_below(p[NPT - 1]), pr = from_above(p[0]);
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) {
+          const T pm = j > 0 ? p[j > 0 ? j - 1 : 0] : pl;
+          const T pp = j < NPT - 1 ? p[j < NPT - 1 ? j + 1 : 0] : pr;
+          const T hh = h[j];
+          const T hgp = (hh * T(-0.5)) * (pm - pp);
+          T F = -hgp - quotient(c6mu * hh * u[j], (T(2) * (hh * hh) + c6d * hh) + c3dd);
+          if constexpr (TH)
+            F = F - noise_node<T>(S.seed, step0 + (uint64_t)s, xw[j]) *
+                        noise_amp(hh, (T)S.kb26, (T)S.delta);
+          if constexpr (EXTRA) {
+            if (S.gg) F = S.gg_sign < 0 ? F - gg[j] : F + gg[j];
+            if (S.body) F = F + (hh * (T)S.alpha) * (T)S.fac;
+          }
+          T e0, e1, e2;
+          if constexpr (usual) {  // feq_node without its terms in g, exact zeros
+            const T uu = u[j] * u[j];
+            e0 = hh * (T(1) - uu);
+            e1 = hh * (T(0.5) * u[j] + T(0.5) * uu);
+            e2 = hh * (T(0.5) * uu - T(0.5) * u[j]);
+          } else {
+            feq_node(hh, u[j], g, e0, e1, e2);
+          }
+          if constexpr (RFT) {
+            h[j] = omeg * t0[j] + itau * e0;
+            u[j] = (omeg * t1[j] + itau * e1) + T(0.5) * F;
+            f2[j] = (omeg * t2[j] + itau * e2) - T(0.5) * F;
+          } else {  // τ = 1: 1/τ = 1 and no f_t
+            h[j] = e0;
+            u[j] = e1 + T(0.5) * F;
+            f2[j] = e2 - T(0.5) * F;
+          }
+        }
+      }
+      // pull-stream (bounce-back at walls) and moments
+      {
+        const T fl = from_below(u[NPT - 1]), fr = from_above(f2[0]);
+        T bl = T(0), br = T(0);
+        if constexpr (EXTRA) {
+          bl = from_below(b1[NPT - 1]);
+          br = from_above(b2[0]);
+        }
+        T prev1 = fl, prevb = bl;  // f1 and b1 of the node before
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) {
+          const T s1 = u[j], s2 = f2[j];
+          const T f0 = h[j];
+          T f1 = prev1, fb = j < NPT - 1 ? f2[j < NPT - 1 ? j + 1 : 0] : fr;
+          if constexpr (EXTRA) {
+            if (walls) {
+              const T bp = j < NPT - 1 ? b2[j < NPT - 1 ? j + 1 : 0] : br;
+              f1 = (f1 - f1 * prevb) + s2 * b2[j];
+              fb = (fb - fb * bp) + s1 * b1[j];
+            }
+            prevb = b1[j];
+          }
+          prev1 = s1;
+          if constexpr (RFT) {
+            t0[j] = f0;
+            t1[j] = f1;
+            t2[j] = fb;
+          }
+          const T hn = (f0 + f1) + fb;
+          h[j] = hn;
+          u[j] = quotient(f1 - fb, hn);
+        }
       }
     }
-  }
+  };
+  if (n == 9 && m == 3 && S.g == 0.0) run(std::true_type{});
+  else run(std::false_type{});
 #pragma unroll
   for (int j = 0; j < NPT; ++j)
     if (j >= own0 && j < own0 + W && xs + j < L) {
@@ -1641,9 +1662,9 @@ hipError_t launch_resident(const Film1* d_table, int nfilms, int64_t nsteps, int
 // SIMD holds one wave (0.24 and 0.22 us with 4 and 8 nodes, whose chains
 // overlap), 0.22 us per node and wave where it holds more.  Fitted to FP64
 // films of 64 to 3e6 nodes over npt 1-8 and k 4-24; the choice is within 7 %
-// of the best pair measured at each (at 1024 nodes (1, 10): 0.51 us a step
-// against 0.64 for (2, 18); at 2e5 (4, 8): 1.50 against 1.69 for (2, 8); at
-// 3e6 (8, 8): 12.2 against 12.5 for (4, 8)).
+// of the best pair measured at each (at 1024 nodes (1, 10): 0.45 us a step
+// against 0.49 for (2, 18); at 2e5 (4, 8): 1.13 against 1.38 for (2, 8); at
+// 3e6 (8, 8): 10.0 against 10.3 for (4, 8)).
 struct WaveShape {
   int npt, k;
 };
@@ -1677,7 +1698,7 @@ void launch_wave_t(const Film1& S, uint64_t step, int k, swalbe::StepSeries ser,
 template <typename T, int NPT>
 void launch_wave_n(const Film1& S, uint64_t step, int k, swalbe::StepSeries ser,
                    hipStream_t st) {
-  const bool extra = S.kap || S.gam || S.gg || S.b1;
+  const bool extra = S.kap || S.gam || S.gg || S.b1 || S.body;
   if (S.read_ft) {
     if (S.thermal)
       extra ? launch_wave_t<T, NPT, true, true, true>(S, step, k, ser, st)
@@ -1727,7 +1748,8 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
     // nodes (threads) per workgroup of k1_step: opts.threads, else 256
     const int nbt = o->threads ? o->threads : 256;
     const int nb = (s->L + nbt * k1_npt(nbt) - 1) / (nbt * k1_npt(nbt));
-    const bool plain = !S.read_ft && !S.thermal && !S.kap && !S.gam && !S.gg && !S.b1;
+    const bool plain =
+        !S.read_ft && !S.thermal && !S.kap && !S.gam && !S.gg && !S.b1 && !S.body;
     const WaveShape shape = wave_shape(s->L, plain ? 8 : 4, 4 * swalbe::device_cus());
     // steps from `it` (1-based) that one launch may take: the last step of the
     // loop is k1_step's; a mass record reads the height before step t = 0 mod
