@@ -1,4 +1,4 @@
-// step_march.hip -- the D2Q9 step of a large film, one wavefront per strip.
+// step_march.hip -- the D2Q9 step of a larger film, one wavefront per strip.
 //
 // A wave owns a strip of 64 columns, one per lane, and marches up a segment of
 // rows.  At output row j it loads h(j+3), forms p(j+2) from h(j+1 .. j+3), the
@@ -21,6 +21,8 @@
 // writes them on every step, stays with the tiles.  Two columns per lane (120
 // written, on 32-byte sectors) were as fast at 4096 x 4096 (106, 204 us) and
 // slower on smaller films (2000 x 1500 FP32 23 us).
+#include <math.h>
+
 #include "step_node.h"
 #include "swalbe_internal.h"
 
@@ -407,20 +409,59 @@ void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
 #undef SW_S
 }
 
-// Four waves per SIMD, which is what the FP64 step holds at once, while that
-// gives segments of up to 32 rows; six for larger films; no segment under 10
-// rows (three more are computed and discarded).  FP64 us per step: 2000 x 1500
-// 36.9 with 13 rows (four), 39.2 with 12; 2500 x 2501 77 with 27 (four), 81
-// with 18; 4096 x 4096 210 with 48 (six), 237 with 71 (four), 242 with 142.
-// Films of fewer than 24 rows of a strip per SIMD are faster in tiles (1024 x
-// 1024 FP32: 18 rows, 12.8 us in strips, 11.8 in tiles; 1200 x 1200: 15.6 and
-// 15.6).
-int march_segment(int Lx, int Ly) {
-  const int64_t simds = 4 * (int64_t)device_cus();
-  const int64_t rows = ((int64_t)(Lx - 1) / kMarchOut + 1) * Ly;
-  if (rows < 24 * simds || Lx < 64 || Ly < 8) return 0;
+// What a step costs: fixed + row us for each row that a wave computes (its
+// segment and `lead` of start-up), times the waves n that share a SIMD, or
+// about `alone` while fewer leave it waiting on a row's chain of operations
+// (joined smoothly).  Up to six waves n is the fullest SIMD's count, beyond it
+// the average and a half.  Fitted to films of 512 x 512 to 4096 x 4096 and
+// segments of 3 to 30 rows, 3-6 % rms.  [double, noise]
+struct MarchCost {
+  double fixed, row, lead, alone;
+};
+constexpr MarchCost kMarchCost[2][2] = {{{3.5, 0.33, 1.0, 1.7}, {4.5, 0.42, 1.1, 1.5}},
+                                        {{2.8, 0.59, 1.7, 1.3}, {4.7, 1.01, 1.7, 1.3}}};
+
+// The segment with the smallest modelled time per step, if that is less than
+// the other path's: with several steps per launch the one modelled there
+// (without noise, which scales both alike), in tiles that or, with noise,
+// 7.5 us and 3.3 us per round of 64 x 8 tiles over the CUs (FP64), 8.6 and
+// 1.25, or 5 and 2.3 beyond four, of 64 x 16 (FP32).  Measured, us per step
+// without / with noise, other path -> strips: FP64 512² 8.5 -> 9.2 / 12.2 ->
+// 13.9, 700 x 640 13.3 -> 11.3 / 20.2 -> 18.8, 850² 20.7 -> 14.0 / 28.8 ->
+// 23.3, 1024² 23.5 -> 18.3 / 34.2 -> 30.1; FP32 700 x 640 9.1 -> 7.9 / 10.9 ->
+// 9.7, 850² 11.9 -> 9.9 / 13.0 -> 12.2, 1024² 11.9 -> 11.5 / 13.5 -> 15.0 (four
+// tiles on every CU), 4000 x 300 15.2 -> 12.1 / 17.1 -> 15.5.
+//
+// Large FP64 films take four waves per SIMD while that gives segments of up to
+// 32 rows, and six beyond: 2500 x 2501 77 us with 28 rows (four), 82 with the
+// 18 of the model; 4096 x 4096 210 with 48 (six), 214 with 24.
+int march_segment(int Lx, int Ly, bool f64, bool noise, const MultiShape& other) {
+  if (Lx < 64 || Ly < 8) return 0;
+  const int64_t cus = device_cus(), simds = 4 * cus;
+  const int64_t strips = (Lx - 1) / kMarchOut + 1, rows = strips * Ly;
   const int64_t four = (rows - 1) / (4 * simds) + 1, six = (rows - 1) / (6 * simds) + 1;
-  return (int)(four > 32 ? six : four < 10 ? 10 : four);
+  if (f64 && four > 16) return (int)(four > 32 ? six : four);
+  double least = other.us;
+  const bool cn = noise && other.geom < 0;
+  if (cn) {
+    const int64_t tiles = (int64_t)((Lx - 1) / 64 + 1) * ((Ly - 1) / (f64 ? 8 : 16) + 1);
+    const double r = (double)((tiles - 1) / cus + 1);
+    least = f64 ? 7.5 + 3.3 * r : r <= 4.0 ? 8.6 + 1.25 * r : 5.0 + 2.3 * r;
+  }
+  const MarchCost& c = kMarchCost[f64][cn];
+  const double a2 = c.alone * c.alone, a4 = a2 * a2;
+  int best = 0;
+  for (int seg = 3; seg <= 64; ++seg) {
+    const int64_t items = strips * ((Ly - 1) / seg + 1);
+    const double n = items <= 6 * simds ? (double)((items - 1) / simds + 1)
+                                        : (double)items / (double)simds + 0.5;
+    const double t = c.fixed + c.row * (seg + c.lead) * sqrt(sqrt(n * n * n * n + a4));
+    if (t < least) {
+      least = t;
+      best = seg;
+    }
+  }
+  return best;
 }
 
 template void launch_march<double>(const StepIO<double>&, const StepParams&, StepSeries, uint64_t,

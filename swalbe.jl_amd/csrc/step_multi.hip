@@ -478,8 +478,8 @@ void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
 
 // The shape with the smallest modelled time per step, unless one launch per
 // step is faster: (FP64) 5.0 us and 2.1 us per round of its 64 x 8 tiles over
-// the CUs, (FP32) 7.6 us and 1.05 us per round of 64 x 16 tiles, when it
-// writes the moments only.  Measured, us per step (several / one per launch):
+// the CUs, (FP32) 7.6 us and 1.05 us per round of 64 x 16 tiles (6 and 1.85
+// beyond four), when it writes the moments only.  Measured, us per step (several / one per launch):
 // FP64 64² 2.32 / 7.48, 256² 3.14 / 7.35, 512² 7.92 / 8.94, 700 x 640 13.9 /
 // 12.7; FP32 64² 2.01 / 8.06, 256² 2.34 / 8.10, 512² 5.32 / 9.04, 850² 11.2 /
 // 11.6, 1024² 14.2 / 11.9.
@@ -489,14 +489,15 @@ MultiShape multi_shape(int Lx, int Ly, bool f64) {
     const int64_t tiles = (int64_t)((Lx - 1) / tx + 1) * ((Ly - 1) / ty + 1);
     return (double)((tiles - 1) / (cus * wgs) + 1);
   };
-  double least = f64 ? 5.0 + 2.1 * rounds(64, 8, 1) : 7.6 + 1.05 * rounds(64, 16, 1);
-  MultiShape best{-1, 1};
+  const double r = rounds(64, f64 ? 8 : 16, 1);
+  double least = f64 ? 5.0 + 2.1 * r : r <= 4.0 ? 7.6 + 1.05 * r : 6.0 + 1.85 * r;
+  MultiShape best{-1, 1, least};
   for (int i = 0; i < kNGeoms; ++i) {
     const Geom& g = f64 ? kGeoms64[i] : kGeoms32[i];
     const double t = (g.fixed + g.body * rounds(g.tx, g.ty, g.wgs)) / g.k;
     if (t < least) {
       least = t;
-      best = MultiShape{i, g.k};
+      best = MultiShape{i, g.k, t};
     }
   }
   return best;

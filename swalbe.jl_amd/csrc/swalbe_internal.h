@@ -260,8 +260,9 @@ void launch_step_f32(const StepIO<float>& io, const StepParams& sp, StepSeries s
 // film, and a launch of k <= shape.k steps; ser: the series slots of the
 // first; write_f: the last of them writes f and p (τ ≠ 1: f always).
 struct MultiShape {
-  int geom;  // -1: one step per launch is the faster path
+  int geom;   // -1: one step per launch is the faster path
   int k;
+  double us;  // the path's modelled time per step without noise
 };
 MultiShape multi_shape(int Lx, int Ly, bool f64);
 template <typename T>
@@ -269,10 +270,11 @@ void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int geom,
                   hipStream_t s);
 
-// One τ = 1 step of a large film, a wave per strip of columns and segment of
+// One τ = 1 step of a larger film, a wave per strip of columns and segment of
 // `seg` rows (step_march.hip), writing the moments, and f and p with write_f.
-// march_segment: the rows per segment for a film, 0 where tiles are faster.
-int march_segment(int Lx, int Ly);
+// march_segment: the rows per segment for a film, 0 where `other` (the path
+// multi_shape chose) is faster.
+int march_segment(int Lx, int Ly, bool f64, bool noise, const MultiShape& other);
 template <typename T>
 void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step,
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int seg, hipStream_t s);
