@@ -1023,8 +1023,9 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
   // materialize_last), and so is every step that something falls between:
   // a mass record or a measurement before step t, a snapshot after it.
   const bool automatic = o->variant == 0 && o->tile_y <= 0;
-  MultiShape multi = automatic ? multi_shape(F.Lx, F.Ly, F.dtype == SWALBE_F64)
-                               : MultiShape{-1, 1, 0.0};
+  MultiShape multi =
+      automatic ? multi_shape(F.Lx, F.Ly, F.dtype == SWALBE_F64, sp.read_ft != 0)
+                : MultiShape{-1, 1, 0.0};
   // larger films whose loop writes f and p on its last step only march in strips
   const int march = automatic && final_only ? march_segment(F.Lx, F.Ly, F.dtype == SWALBE_F64,
                                                             sp.thermal != 0, multi)

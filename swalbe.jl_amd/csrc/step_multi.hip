@@ -1,5 +1,6 @@
 // step_multi.hip -- several D2Q9 steps of one film per launch, for films too
-// small to fill the chip one step at a time.
+// small to fill the chip one step at a time, and for FP32 films whose carried
+// populations (τ ≠ 1) outgrow the caches.
 //
 // A workgroup owns a TX x TY tile and stages it with a halo of 3 K nodes in
 // LDS; a step costs three nodes of halo at each side (one per stencil), so
@@ -483,7 +484,7 @@ void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
 // FP64 64² 2.32 / 7.48, 256² 3.14 / 7.35, 512² 7.92 / 8.94, 700 x 640 13.9 /
 // 12.7; FP32 64² 2.01 / 8.06, 256² 2.34 / 8.10, 512² 5.32 / 9.04, 850² 11.2 /
 // 11.6, 1024² 14.2 / 11.9.
-MultiShape multi_shape(int Lx, int Ly, bool f64) {
+MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried) {
   const int64_t cus = device_cus();
   auto rounds = [&](int tx, int ty, int wgs) {
     const int64_t tiles = (int64_t)((Lx - 1) / tx + 1) * ((Ly - 1) / ty + 1);
@@ -500,6 +501,13 @@ MultiShape multi_shape(int Lx, int Ly, bool f64) {
       best = MultiShape{i, g.k, t};
     }
   }
+  // FP32 films that carry their populations (τ ≠ 1) outgrow the caches, where
+  // two steps per launch halve the traffic of the 18 planes.  us per step, one
+  // / two steps: 1000 x 1031 24.5 / 23.8, 1200² 32.7 / 33.5, 1300 x 1250 44.5 /
+  // 35.8, 2000 x 1500 78 / 64, 3000² 256 / 180, 4096² 389 / 323, with noise 397
+  // / 355.  FP64 tiles are bound by arithmetic: 2000 x 1500 118 / 141.
+  if (carried && !f64 && best.geom < 0 && (int64_t)Lx * Ly >= 1600000)
+    best = MultiShape{3, kGeoms32[3].k, least};
   return best;
 }
 

@@ -264,7 +264,7 @@ struct MultiShape {
   int k;
   double us;  // the path's modelled time per step without noise
 };
-MultiShape multi_shape(int Lx, int Ly, bool f64);
+MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried);
 template <typename T>
 void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step, int k,
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int geom,
