@@ -661,11 +661,11 @@ extern "C" int swalbe_step_advance(swalbe_state* st, double g, double tau) {
 
 // ---------------------------------------------------------------- reductions
 static int reduce_enqueue(swalbe_state* st, const void* p, double href, double thresh,
-                          double* out_dev) {
+                          double* out_dev, uint32_t* flag = nullptr, uint32_t seq = 0) {
   Film& F = st->film;
   SW_BOTH(st, launch_reduce<T>((const T*)p, F.N, href, thresh, st->partials, st->nparts,
                                st->stream));
-  launch_reduce_finish(st->partials, st->nparts, out_dev, st->stream);
+  launch_reduce_finish(st->partials, st->nparts, out_dev, st->stream, flag, seq);
   SW_HIP(hipGetLastError());
   return SWALBE_OK;
 }
@@ -686,7 +686,9 @@ int swalbe_reduce(swalbe_state* st, int32_t field, double thresh, double out[4])
   HostResult res(st->device, st->stream);
   // four doubles straight into pinned memory; without any, through the device
   double* dst = res.dev() ? res.dev() : st->red_out;
-  if (int rc = reduce_enqueue(st, p, enc_offset(st->film, field, 0), thresh, dst)) return rc;
+  if (int rc = reduce_enqueue(st, p, enc_offset(st->film, field, 0), thresh, dst, res.flag(),
+                              res.seq()))
+    return rc;
   if (!res.dev())
     SW_HIP(hipMemcpyAsync(out, dst, 4 * sizeof(double), hipMemcpyDeviceToHost, st->stream));
   SW_HIP(res.get(out, 4));

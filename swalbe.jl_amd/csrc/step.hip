@@ -574,7 +574,7 @@ __global__ void k_reduce(const T* __restrict__ h, int64_t N, double href, double
 // 1024 partials, each load waiting for the last, took 169 us at 4096 x 4096;
 // the wave takes 6.)
 __global__ void k_reduce_finish(const double* __restrict__ partials, int nparts,
-                                double* __restrict__ out) {
+                                double* __restrict__ out, uint32_t* flag, uint32_t seq) {
   double sum = 0.0, mx = -__builtin_inf(), mn = __builtin_inf(), cnt = 0.0;
   for (int i = threadIdx.x; i < nparts; i += 64) {
     const double a = partials[4 * i + 1], b = partials[4 * i + 2];
@@ -595,6 +595,8 @@ __global__ void k_reduce_finish(const double* __restrict__ partials, int nparts,
   out[1] = mx;
   out[2] = mn;
   out[3] = cnt;
+  if (!flag) return;
+  __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace
@@ -615,8 +617,9 @@ void launch_reduce(const T* h, int64_t N, double href, double thresh, double* pa
                      partials);
 }
 
-void launch_reduce_finish(const double* partials, int nparts, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, partials, nparts, out);
+void launch_reduce_finish(const double* partials, int nparts, double* out, hipStream_t s,
+                          uint32_t* flag, uint32_t seq) {
+  hipLaunchKernelGGL(k_reduce_finish, dim3(1), dim3(64), 0, s, partials, nparts, out, flag, seq);
 }
 
 SeriesRun::~SeriesRun() {

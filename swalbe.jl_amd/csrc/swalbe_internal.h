@@ -283,7 +283,9 @@ void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
 template <typename T>
 void launch_reduce(const T* h, int64_t N, double href, double thresh, double* partials,
                    int nparts, hipStream_t s);
-void launch_reduce_finish(const double* partials, int nparts, double* out, hipStream_t s);
+// flag (with out in pinned host memory): set to seq behind the results
+void launch_reduce_finish(const double* partials, int nparts, double* out, hipStream_t s,
+                          uint32_t* flag = nullptr, uint32_t seq = 0);
 
 // On-device measurements of a height field (href added to every value):
 // out = {count(h > thresh), max h, Σ sqrt(|∇h|² + 1) over h > thresh,
@@ -308,17 +310,19 @@ int field_from_host(void* dev, size_t des, const void* host, size_t hes, int64_t
 void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const double* from,
                      const double* to, hipStream_t s);
 // A few doubles that a kernel writes straight into pinned host memory: pass
-// dev() to the kernel, then get() waits for the stream and copies them out.
-// dev() is null where no pinned memory is to be had.
+// dev(), flag() and seq() (called once) to the kernel, which sets the flag to
+// seq behind the data; then get() waits for it and copies them out.  dev() and
+// flag() are null where no pinned memory is to be had.
 class HostResult {
  public:
   HostResult(int device, hipStream_t s);
   ~HostResult();
   double* dev() const { return p_; }
+  uint32_t* flag() const;
+  uint32_t seq();
   hipError_t get(double* out, int n);
 
  private:
-  int device_;
   hipStream_t s_;
   void* stage_ = nullptr;
   double* p_ = nullptr;

@@ -13,8 +13,10 @@
 #include <string.h>
 
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "swalbe_internal.h"
@@ -36,9 +38,27 @@ inline int copy_threads(size_t bytes) {
 // ---------------------------------------------------------------- pinned buffers
 struct Stage {
   int device = 0;
-  char* pin = nullptr;
+  char* pin = nullptr;  // kChunk bytes and the flag behind them
   hipEvent_t ev = nullptr;
+  uint32_t seq = 0;  // the flag's value after the buffer's last flagged kernel
+
+  uint32_t* flag() const { return (uint32_t*)(pin + kChunk); }
 };
+
+// Waits for a kernel that ends by setting its buffer's flag: polls for up to
+// 100 us, which is quicker by 5 us than waiting for the stream, then waits for
+// the stream (which also reports a kernel that failed).
+hipError_t flag_wait(const Stage& st, hipStream_t s) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    for (int i = 0; i < 64; ++i) {
+      if (__atomic_load_n(st.flag(), __ATOMIC_ACQUIRE) == st.seq) return hipSuccess;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(100))
+      return hipStreamSynchronize(s);
+  }
+}
 
 void stage_free(Stage& s) {
   if (s.ev) (void)hipEventDestroy(s.ev);
@@ -71,8 +91,9 @@ hipError_t stage_take(int device, Stage* out) {
   }
   Stage s;
   s.device = device;
-  hipError_t e = hipHostMalloc((void**)&s.pin, kChunk,
+  hipError_t e = hipHostMalloc((void**)&s.pin, kChunk + 64,
                                hipHostMallocPortable | hipHostMallocCoherent);
+  if (e == hipSuccess) *s.flag() = 0;
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s.ev, hipEventDisableTiming);
   if (e != hipSuccess) {
     stage_free(s);
@@ -160,6 +181,38 @@ __global__ __launch_bounds__(256) void k_reencode(float* __restrict__ dev, int64
   }
 }
 
+// A small field in one workgroup, which tells the host by a flag behind the
+// data.  A download of 1024 doubles takes 9.9 us instead of 15.2 with a wait for
+// the stream, an upload 10.8 instead of 16; at 4096 12 and 15, at 8192 one
+// workgroup is no faster.
+constexpr int64_t kSmall = 4096;  // elements
+
+template <typename TD, typename TH, bool BITS, bool DOWN>
+__global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __restrict__ pin,
+                                                int planes, int64_t n, int64_t stride,
+                                                Offsets off, uint32_t* flag, uint32_t seq) {
+  for (int k = 0; k < planes; ++k) {
+    const double o = off.v[k];
+    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+      if constexpr (BITS) {
+        if constexpr (DOWN) pin[k * n + i] = dev[k * stride + i];
+        else dev[k * stride + i] = pin[k * n + i];
+      } else if constexpr (DOWN) {
+        const double v = (double)dev[k * stride + i];
+        pin[k * n + i] = (TH)(o == 0.0 ? v : v + o);
+      } else {
+        dev[k * stride + i] = (TD)((double)pin[k * n + i] - o);
+      }
+    }
+  }
+  // every wave's stores have left before the flag's release, which writes the
+  // L2 back for all of them (a fence at workgroup scope waits for none)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 Offsets offsets(const double* off, int planes) {
   Offsets o{};
   for (int k = 0; off && k < planes; ++k) o.v[k] = off[k];
@@ -176,11 +229,22 @@ struct Job {
   int planes, device;
   Offsets off;
   bool bits;
+  bool small;   // one workgroup and a flag (k_small)
   bool single;  // one chunk: its end is the stream's, no event (0.9 us less of 16)
   hipStream_t s;
   std::atomic<int64_t> next{0};
   std::atomic<int> err{0};
 };
+
+template <typename TD, typename TH, bool BITS>
+void launch_small(const Job& J, const Stage& st) {
+  if (J.down)
+    hipLaunchKernelGGL((k_small<TD, TH, BITS, true>), dim3(1), dim3(1024), 0, J.s, (TD*)J.dev,
+                       (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
+  else
+    hipLaunchKernelGGL((k_small<TD, TH, BITS, false>), dim3(1), dim3(1024), 0, J.s, (TD*)J.dev,
+                       (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
+}
 
 template <typename TD, typename TH, bool BITS>
 void launch_piece(const Job& J, char* pin, const Piece& P, dim3 grid) {
@@ -192,20 +256,32 @@ void launch_piece(const Job& J, char* pin, const Piece& P, dim3 grid) {
                        (const TH*)pin, P, J.off);
 }
 
+// f(TD, TH, BITS) as types, for the job's elements
+template <typename F>
+void with_types(const Job& J, F&& f) {
+  if (J.bits) {
+    if (J.des == 8) f(uint64_t{}, uint64_t{}, std::true_type{});
+    else f(uint32_t{}, uint32_t{}, std::true_type{});
+  } else if (J.des == 8) {
+    if (J.hes == 8) f(double{}, double{}, std::false_type{});
+    else f(double{}, float{}, std::false_type{});
+  } else {
+    if (J.hes == 8) f(float{}, double{}, std::false_type{});
+    else f(float{}, float{}, std::false_type{});
+  }
+}
+
 hipError_t issue(const Job& J, Stage& st, int64_t a, int64_t b) {
   Piece P{a, b, J.n, J.stride, (int)(a / J.n)};
   const int64_t widest = b - a < J.n ? b - a : J.n;
   const dim3 grid((unsigned)((widest + 255) / 256), (unsigned)((b - 1) / J.n - a / J.n + 1));
-  if (J.bits) {
-    if (J.des == 8) launch_piece<uint64_t, uint64_t, true>(J, st.pin, P, grid);
-    else launch_piece<uint32_t, uint32_t, true>(J, st.pin, P, grid);
-  } else if (J.des == 8) {
-    if (J.hes == 8) launch_piece<double, double, false>(J, st.pin, P, grid);
-    else launch_piece<double, float, false>(J, st.pin, P, grid);
-  } else {
-    if (J.hes == 8) launch_piece<float, double, false>(J, st.pin, P, grid);
-    else launch_piece<float, float, false>(J, st.pin, P, grid);
-  }
+  if (J.small) ++st.seq;
+  with_types(J, [&](auto td, auto th, auto bits) {
+    using TD = decltype(td);
+    using TH = decltype(th);
+    if (J.small) launch_small<TD, TH, decltype(bits)::value>(J, st);
+    else launch_piece<TD, TH, decltype(bits)::value>(J, st.pin, P, grid);
+  });
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && !J.single) e = hipEventRecord(st.ev, J.s);
   return e;
@@ -220,7 +296,9 @@ void run_chunks(Job* pJ) {
   hipError_t e = hipSetDevice(J.device);
   auto finish = [&](int r) {  // wait for buffer r; a download's chunk goes to the caller
     if (b[r] < 0) return;
-    const hipError_t w = J.single ? hipStreamSynchronize(J.s) : hipEventSynchronize(st[r].ev);
+    const hipError_t w = J.small    ? flag_wait(st[r], J.s)
+                         : J.single ? hipStreamSynchronize(J.s)
+                                    : hipEventSynchronize(st[r].ev);
     if (w == hipSuccess && J.down && e == hipSuccess)
       memcpy(J.host + (size_t)a[r] * J.hes, st[r].pin, (size_t)(b[r] - a[r]) * J.hes);
     if (e == hipSuccess) e = w;
@@ -264,6 +342,7 @@ int transfer(bool down, void* host, size_t hes, void* dev, size_t des, int64_t n
   J.total = n * planes;
   J.per = (int64_t)(kChunk / hes);
   J.single = J.total <= J.per;
+  J.small = J.total <= kSmall;
   J.device = device;
   J.off = offsets(off, planes);
   J.bits = hes == des;
@@ -302,7 +381,7 @@ void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const do
                      dim3(256), 0, s, dev, n, stride, offsets(from, planes), offsets(to, planes));
 }
 
-HostResult::HostResult(int device, hipStream_t s) : device_(device), s_(s) {
+HostResult::HostResult(int device, hipStream_t s) : s_(s) {
   Stage* st = new Stage;
   if (stage_take(device, st) != hipSuccess) (void)hipGetLastError();
   stage_ = st;
@@ -311,14 +390,19 @@ HostResult::HostResult(int device, hipStream_t s) : device_(device), s_(s) {
 
 HostResult::~HostResult() {
   Stage* st = (Stage*)stage_;
-  // whatever was launched may still write: the buffer goes back when it cannot
-  if (st->pin) (void)hipStreamSynchronize(s_);
+  // a kernel launched without get() may still write: the buffer goes back when
+  // it cannot
+  if (st->pin && __atomic_load_n(st->flag(), __ATOMIC_ACQUIRE) != st->seq)
+    (void)hipStreamSynchronize(s_);
   stage_give(*st);
   delete st;
 }
 
+uint32_t* HostResult::flag() const { return p_ ? ((Stage*)stage_)->flag() : nullptr; }
+uint32_t HostResult::seq() { return ++((Stage*)stage_)->seq; }
+
 hipError_t HostResult::get(double* out, int n) {
-  const hipError_t e = hipStreamSynchronize(s_);
+  const hipError_t e = p_ ? flag_wait(*(Stage*)stage_, s_) : hipStreamSynchronize(s_);
   if (e == hipSuccess && p_) memcpy(out, p_, sizeof(double) * (size_t)n);
   return e;
 }

@@ -1,4 +1,4 @@
-"""Fields between host arrays and the device: chunks of 1 MiB through pinned
+"""Fields between host arrays and the device: chunks of 512 KiB through pinned
 buffers, converted on the GPU.  Every value must arrive as the plain formula
 gives it (FP32 states hold float32(v - offset) and give back that plus the
 offset in FP64), at the edges of a chunk, across planes and with one, two and
@@ -19,7 +19,7 @@ def S():
     return swalbe
 
 
-# 131072 doubles (262144 floats) fill a chunk; 1048576 doubles are 8 MiB (four threads)
+# 65536 doubles (131072 floats) fill a chunk; 1048576 doubles are 8 MiB (four threads)
 SHAPES = [(1, 1), (7, 5), (512, 256), (513, 256), (511, 257), (1024, 1025), (1153, 911)]
 
 
