@@ -487,7 +487,7 @@ __device__ __forceinline__ T from_above(T v) {
 // steps.  Measured against the kernels it replaces for single films (us per
 // step): L = 1024 4.6 in one workgroup's LDS -> 0.45, over up to 256 CUs
 // instead of one; L = 3e6 36.4 with one launch and 64 bytes per node and step
-// -> 10.0, with 6 bytes per node and step.
+// -> 10.3, with 6 bytes per node and step.
 // The loop exists twice: for the usual law, n = 9, m = 3 and g = 0, without a
 // branch per node, so that the division chains of a lane's nodes overlap, and
 // for any other (one copy with the branches and the compiler's division: 0.51
@@ -1664,7 +1664,7 @@ hipError_t launch_resident(const Film1* d_table, int nfilms, int64_t nsteps, int
 // films of 64 to 3e6 nodes over npt 1-8 and k 4-24; the choice is within 7 %
 // of the best pair measured at each (at 1024 nodes (1, 10): 0.45 us a step
 // against 0.49 for (2, 18); at 2e5 (4, 8): 1.13 against 1.38 for (2, 8); at
-// 3e6 (8, 8): 10.0 against 10.3 for (4, 8)).
+// 3e6 (4, 4): 10.3, the best pair (8, 8) 10.0).
 struct WaveShape {
   int npt, k;
 };

@@ -309,7 +309,7 @@ __global__ void k_force_sum(T* __restrict__ Fx, T* __restrict__ Fy, const T* __r
 // equilibrium! runs these instead of five and three op kernels: every field
 // an op would write is written, with its bits, and a step costs two launches.
 // A step of 512 x 512 FP64 with a reduction in the callback took 88 us with
-// the eight op kernels (45 us of GPU time); with these two it takes 47 (24).
+// the eight op kernels (45 us of GPU time); with these two it takes 40 (24).
 
 // filmpressure!, h∇p!, slippage!, [thermal!] and the force sum.  A workgroup
 // takes 64 x kFY nodes; their pressures and a ring around them go through LDS.
