@@ -15,6 +15,7 @@
 #include <atomic>
 #include <chrono>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -382,14 +383,15 @@ void launch_reencode(float* dev, int64_t n, int planes, int64_t stride, const do
 }
 
 HostResult::HostResult(int device, hipStream_t s) : s_(s) {
-  Stage* st = new Stage;
-  if (stage_take(device, st) != hipSuccess) (void)hipGetLastError();
+  Stage* st = new (std::nothrow) Stage;
+  if (st && stage_take(device, st) != hipSuccess) (void)hipGetLastError();
   stage_ = st;
-  p_ = (double*)st->pin;
+  p_ = st ? (double*)st->pin : nullptr;
 }
 
 HostResult::~HostResult() {
   Stage* st = (Stage*)stage_;
+  if (!st) return;
   // a kernel launched without get() may still write: the buffer goes back when
   // it cannot
   if (st->pin && __atomic_load_n(st->flag(), __ATOMIC_ACQUIRE) != st->seq)
@@ -399,7 +401,7 @@ HostResult::~HostResult() {
 }
 
 uint32_t* HostResult::flag() const { return p_ ? ((Stage*)stage_)->flag() : nullptr; }
-uint32_t HostResult::seq() { return ++((Stage*)stage_)->seq; }
+uint32_t HostResult::seq() { return p_ ? ++((Stage*)stage_)->seq : 0; }
 
 hipError_t HostResult::get(double* out, int n) {
   const hipError_t e = p_ ? flag_wait(*(Stage*)stage_, s_) : hipStreamSynchronize(s_);
