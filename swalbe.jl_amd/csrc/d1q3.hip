@@ -482,12 +482,12 @@ __device__ __forceinline__ T from_above(T v) {
 // output.
 //
 // What bounds it: FP64 issue (about 85 instructions per node and step, three
-// correctly rounded divisions among them).  One node per lane takes 0.25 us a
-// step however short the film; the 2.2 us of a launch are shared by its k
+// correctly rounded divisions among them).  One node per lane takes 0.2 us a
+// step however short the film; the 2.9 us of a launch are shared by its k
 // steps.  Measured against the kernels it replaces for single films (us per
-// step): L = 1024 4.6 in one workgroup's LDS -> 0.45, over up to 256 CUs
+// step): L = 1024 4.6 in one workgroup's LDS -> 0.47, over up to 256 CUs
 // instead of one; L = 3e6 36.4 with one launch and 64 bytes per node and step
-// -> 10.3, with 6 bytes per node and step.
+// -> 9.2, with 5 bytes per node and step.
 // The loop exists twice: for the usual law, n = 9, m = 3 and g = 0, without a
 // branch per node, so that the division chains of a lane's nodes overlap, and
 // for any other (one copy with the branches and the compiler's division: 0.51
@@ -1656,34 +1656,39 @@ hipError_t launch_resident(const Film1* d_table, int nfilms, int64_t nsteps, int
 }
 
 // Nodes per lane and steps per launch of k1_wave for a film of L nodes: the
-// pair with the smallest modelled time per step.  A launch costs 1.2 us and
-// 0.5 us per node of a lane (its strided loads and stores), 0.8 us more where
-// a SIMD takes more than one wave; a step 0.28 us per node of a lane while a
-// SIMD holds one wave (0.24 and 0.22 us with 4 and 8 nodes, whose chains
-// overlap), 0.22 us per node and wave where it holds more.  Fitted to FP64
-// films of 64 to 3e6 nodes over npt 1-8 and k 4-24; the choice is within 7 %
-// of the best pair measured at each (at 1024 nodes (1, 10): 0.45 us a step
-// against 0.49 for (2, 18); at 2e5 (4, 8): 1.13 against 1.38 for (2, 8); at
-// 3e6 (4, 4): 10.3, the best pair (8, 8) 10.0).
+// pair with the smallest modelled time per step.  A launch costs 2.57 us, 0.32
+// per node of a lane and 0.14 per node and further wave on a SIMD; a step 0.142
+// us per node of a lane times the waves that share a SIMD, or times about
+// `alone` where they are fewer and wait on a node's chain of operations (joined
+// smoothly; up to six waves the fullest SIMD's count, beyond it the average and
+// a half).  Fitted to FP64 films of 1024 to 4e6 nodes over npt 1-8 and k 2-24,
+// 3.5 % rms; the choice is within 2 % of the best pair measured at each from
+// 65000 nodes up.  us per step: 1024 nodes (1, 10) 0.47, (2, 16) 0.53; 20000
+// (2, 16) 0.55, (1, 6) 0.69; 2e5 (4, 10) 1.05, (2, 10) 1.31; 1e6 (4, 10) 3.6,
+// (8, 24) 3.8; 3e6 (8, 10) 9.2, (4, 4) 9.8; 4e6 (8, 10) 11.8, (4, 4) 13.0.
 struct WaveShape {
   int npt, k;
 };
 WaveShape wave_shape(int L, int most, int simds) {
   WaveShape best{1, 1};
   double least = 1e30;
-  for (int npt = 1; npt <= most; npt *= 2)
+  for (int npt = 1; npt <= most; npt *= 2) {
+    const double alone = npt == 1 ? 1.29 : npt == 2 ? 1.15 : npt == 4 ? 0.80 : 0.88;
+    const double a4 = alone * alone * alone * alone;
     for (int k = 2; k <= 32; k += 2) {
       const int W = 64 * npt - 6 * k;
       if (W < 4) break;
-      const int per = (int)(((int64_t)(L - 1) / W + simds) / simds);  // waves per SIMD
-      const double alone = npt <= 2 ? 0.28 : npt == 4 ? 0.24 : 0.22;
-      const double node = per == 1 ? alone : std::max(alone, 0.22 * per);
-      const double t = (1.2 + 0.5 * npt + (per > 1 ? 0.8 : 0.0)) / k + npt * node;
+      const int64_t waves = (L - 1) / W + 1;
+      const double n = waves <= 6 * (int64_t)simds ? (double)((waves - 1) / simds + 1)
+                                                   : (double)waves / simds + 0.5;
+      const double t = (2.57 + npt * (0.32 + 0.14 * (n - 1.0))) / k +
+                       0.142 * npt * sqrt(sqrt(n * n * n * n + a4));
       if (t < least) {
         least = t;
         best = WaveShape{npt, k};
       }
     }
+  }
   return best;
 }
 
