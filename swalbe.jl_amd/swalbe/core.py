@@ -722,17 +722,19 @@ def _time_loop_callback(sys, state, f: Callable, measure, verbose, thermal, seed
     """Op-by-op loop for an arbitrary measurement callback
     (src/simulate.jl:69-96): the ops before f in one call, those after it in
     another, every field of the state written as the single ops would.  f may
-    change the state and sys.param."""
+    change the state, change sys.param or replace it; the ops take sys.param
+    as it is when they run, the noise the one that the loop began with."""
     P = sys.param
     L = lib()
     for _ in range(P.Tmax):
         t = state.t + 1
         if P.tdump > 0 and t % P.tdump == 0 and verbose:
             print(f"Time step {t} mass is {round(state.reduce()['sum'], 3)}")
-        if np.ndim(P.θ) == 0:
-            check(L.swalbe_step_forces(state.handle, C.byref(P.cparams()), int(bool(thermal)),
+        Q = sys.param
+        if np.ndim(Q.θ) == 0 and (Q is P or not thermal):
+            check(L.swalbe_step_forces(state.handle, C.byref(Q.cparams()), int(bool(thermal)),
                                        int(seed), int(t)), "step_forces")
-        else:  # f made θ a field
+        else:  # θ is a field, or the noise has other parameters than the rest
             filmpressure(state, sys)
             h_grad_p(state)
             slippage(state, sys)
@@ -740,6 +742,7 @@ def _time_loop_callback(sys, state, f: Callable, measure, verbose, thermal, seed
                 check(L.swalbe_thermal(state.handle, P.kbt, P.μ, P.δ, int(seed), int(t)), "thermal")
             force_sum(state, thermal)
         f(measure, state)
-        check(L.swalbe_step_advance(state.handle, float(P.g), float(P.τ)), "step_advance")
+        Q = sys.param
+        check(L.swalbe_step_advance(state.handle, float(Q.g), float(Q.τ)), "step_advance")
         state.t = t
     return state, measure
