@@ -24,6 +24,8 @@
 
 using swalbe::dkey;
 using swalbe::dkey_inv;
+using swalbe::kNoMax;
+using swalbe::kNoMin;
 using swalbe::hip_fail;
 using swalbe::kTagThermal;
 using swalbe::normal_pair;
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step, swalbe::St
   const T* b1 = (const T*)S.b1;
   const T* b2 = (const T*)S.b2;
   T* fout = (T*)S.f_out;
-  unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
+  unsigned long long kmax = kNoMax, kmin = kNoMin, cnt = 0ull;
 #pragma unroll
   for (int q = 0; q < NPT; ++q) {
     const int j = t + q * NB;  // output node x0 + j
@@ -400,9 +402,11 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step, swalbe::St
     if (x >= L) break;
     if (ser.base) {
       const double hv = (double)sh[j + 3];
-      const unsigned long long k = dkey(hv);
-      kmax = k > kmax ? k : kmax;
-      kmin = k < kmin ? k : kmin;
+      if (hv == hv || !ser.skip_nan) {
+        const unsigned long long k = dkey(hv);
+        kmax = k > kmax ? k : kmax;
+        kmin = k < kmin ? k : kmin;
+      }
       cnt += hv > S.wet_thresh ? 1ull : 0ull;
     }
     const int xm = x == 0 ? L - 1 : x - 1, xp = x == L - 1 ? 0 : x + 1;
@@ -543,14 +547,16 @@ __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, in
 #pragma unroll 1
     for (int s = 0; s < k; ++s) {
       if (ser.base) {  // series over the step's input height
-        unsigned long long kmax = 0ull, kmin = ~0ull, cnt = 0ull;
+        unsigned long long kmax = kNoMax, kmin = kNoMin, cnt = 0ull;
 #pragma unroll
         for (int j = 0; j < NPT; ++j)
           if (j >= own0 && j < own0 + W && xs + j < L) {
             const double hv = (double)h[j];
-            const unsigned long long q = dkey(hv);
-            kmax = q > kmax ? q : kmax;
-            kmin = q < kmin ? q : kmin;
+            if (hv == hv || !ser.skip_nan) {
+              const unsigned long long q = dkey(hv);
+              kmax = q > kmax ? q : kmax;
+              kmin = q < kmin ? q : kmin;
+            }
             cnt += hv > S.wet_thresh ? 1ull : 0ull;
           }
         for (int o = 32; o > 0; o >>= 1) {
@@ -1755,6 +1761,7 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
     const int nb = (s->L + nbt * k1_npt(nbt) - 1) / (nbt * k1_npt(nbt));
     const bool plain =
         !S.read_ft && !S.thermal && !S.kap && !S.gam && !S.gg && !S.b1 && !S.body;
+    const bool fits = fits_resident(s, p);
     const WaveShape shape = wave_shape(s->L, plain ? 8 : 4, 4 * swalbe::device_cus());
     // steps from `it` (1-based) that one launch may take: the last step of the
     // loop is k1_step's; a mass record reads the height before step t = 0 mod
@@ -1782,7 +1789,9 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
                                    mass + 4 * km, s->stream));
         ++km;
       }
-      const swalbe::StepSeries ser = series.at(it - 1);
+      swalbe::StepSeries ser = series.at(it - 1);
+      // a film that k1_resident could take has its series: NaN heights passed over
+      ser.skip_nan = wave && fits;
       if (wave && it < nsteps)
         SW_BOTH1(s, launch_wave<T>(S, (uint64_t)t, shape.npt, (int)k, ser, s->stream));
       else if (nbt == 1024)

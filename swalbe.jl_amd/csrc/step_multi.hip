@@ -119,15 +119,15 @@ struct Multi {
       }
   }
 
-  // max, min and count(> thresh) of the step's input height over the tile's nodes, gathered by
+  // max, min and count(> thresh) of the step's input height over the tile's nodes (NaN passed
+  // over, as k_step's comparisons do; nothing but NaN: -inf and inf), gathered by
   // LDS atomics that nobody waits for before the next barrier (a shuffle tree per wave and one
   // thread walking the waves' results took 1.2 us a step, half a step of a 100 x 100 film);
   // eight addresses share the lanes of a wave
   __device__ __forceinline__ void series(unsigned long long* red) const {
     using I = Inner<RW, RH, 3 * K, NT>;
-    unsigned long long kmax = 0ull, kmin = ~0ull;
+    unsigned long long kmax = kNoMax, kmin = kNoMin;
     unsigned int cnt = 0;
-    bool any = false;
 #pragma unroll
     for (int q = 0; q < I::NQ; ++q) {
       const int o = I::off(q);
@@ -137,14 +137,15 @@ struct Multi {
       if (own) {
         hv = (double)plane(kH)[o];
         if constexpr (F32) hv = (double)K32.href + hv;
-        const unsigned long long key = dkey(hv);
-        kmax = key > kmax ? key : kmax;
-        kmin = key < kmin ? key : kmin;
-        any = true;
+        if (hv == hv) {
+          const unsigned long long key = dkey(hv);
+          kmax = key > kmax ? key : kmax;
+          kmin = key < kmin ? key : kmin;
+        }
       }
       cnt += (unsigned int)__popcll(__ballot(own && hv > sp.wet_thresh));
     }
-    if (R.ser.dh && any) {
+    if (R.ser.dh && kmax >= kmin) {
       atomicMax(&red[2 * (threadIdx.x & 7)], kmax);
       atomicMin(&red[2 * (threadIdx.x & 7) + 1], kmin);
     }
@@ -155,7 +156,7 @@ struct Multi {
   // next step's series comes after two more barriers)
   __device__ __forceinline__ void series_out(unsigned long long* red, int64_t i) const {
     if (threadIdx.x != 0) return;
-    unsigned long long kmax = 0ull, kmin = ~0ull;
+    unsigned long long kmax = kNoMax, kmin = kNoMin;
     if (R.ser.dh)
       for (int w = 0; w < 8; ++w) {
         kmax = red[2 * w] > kmax ? red[2 * w] : kmax;
@@ -166,8 +167,8 @@ struct Multi {
   }
   static __device__ __forceinline__ void series_clear(unsigned long long* red) {
     for (int w = 0; w < 8; ++w) {
-      red[2 * w] = 0ull;
-      red[2 * w + 1] = ~0ull;
+      red[2 * w] = kNoMax;
+      red[2 * w + 1] = kNoMin;
     }
     red[16] = 0ull;
   }

@@ -195,9 +195,12 @@ StepParams make_step_params(const swalbe_params* p, const swalbe_step_opts* o, i
 // serialises at 7 ns per workgroup (256 x 256: 3.3 us a step of 256 tiles
 // against 3.1 for the step itself; 1024 x 1024: 33 us of 2048 tiles).
 constexpr int kSeriesSlots = 32, kSeriesWords = 16;
+// keys of -inf and inf: the maximum and minimum of no value (every height NaN)
+constexpr unsigned long long kNoMax = 0x000fffffffffffffull, kNoMin = 0xfff0000000000000ull;
 struct StepSeries {
   unsigned long long* base;  // the (first) step's slots: words max key, min key, count; or null
   int dh, wet;               // which of them are wanted
+  int skip_nan = 0;          // 1D kernels: pass over NaN heights (else the largest of all)
   __device__ __forceinline__ unsigned long long* slot(int64_t step) const {
     return base + (step * kSeriesSlots + (blockIdx.x & (kSeriesSlots - 1))) * kSeriesWords;
   }
