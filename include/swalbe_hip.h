@@ -202,8 +202,9 @@ typedef struct swalbe_step_opts {
     /* 1: with τ = 1, write the distributions and the pressure on the last
      * step only (no step reads them, so every result is the same); the
      * other fields are written every step.  Ignored when τ ≠ 1.  With
-     * variant = 0 and tile_y = 0 large films then run a kernel of their own:
-     * the same FP64 bits, FP32 to rounding. */
+     * variant = 0 and tile_y = 0 large films then run a kernel of their own,
+     * loops of a few steps excepted (swalbe_loop_kernel): the same FP64 bits,
+     * FP32 to rounding. */
     int32_t final_outputs_only;
 } swalbe_step_opts;
 int swalbe_time_loop(swalbe_state *st, const swalbe_params *p, int64_t nsteps,
@@ -212,6 +213,13 @@ int swalbe_time_loop(swalbe_state *st, const swalbe_params *p, int64_t nsteps,
  * the nsteps launches measured with HIP events on the state's stream. */
 int swalbe_time_loop_timed(swalbe_state *st, const swalbe_params *p, int64_t nsteps,
                            const swalbe_step_opts *opts, double *ms_out);
+/* The kernel that swalbe_time_loop takes for this film, loop length and
+ * options: out = {0: one step per launch in tiles, 1: several steps per launch
+ * from LDS, 2: strips; the tile shape's number (1) or the rows per segment (2);
+ * the most steps of a launch; 1 if steps that these kernels are slower at (the
+ * last, those alone in a launch) go to the tiles}. */
+int swalbe_loop_kernel(swalbe_state *st, const swalbe_params *p, int64_t nsteps,
+                       const swalbe_step_opts *opts, int32_t out[4]);
 
 /* ---- reductions: sum(state.height) (src/simulate.jl:10), maximum/minimum
  * (:56) and count(h .> thresh) (src/measures.jl:13-17), in FP64.

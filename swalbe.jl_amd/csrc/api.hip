@@ -838,6 +838,29 @@ struct LoopBuffers {
   }
 };
 
+// The kernels of one loop.
+struct LoopPlan {
+  MultiShape multi;  // geom >= 0: up to multi.k steps per launch
+  int march;         // > 0: strips in segments of so many rows
+  // launches of the one-step tiles in between (the same FP64 bits)
+  bool single_tiles;  // a launch of one step, of a film that takes several
+  bool last_tiles;    // the step that writes f and p, of a film that takes strips
+};
+
+LoopPlan loop_plan(const Film& F, const StepParams& sp, const swalbe_step_opts* o, int64_t nsteps,
+                   bool final_only) {
+  const bool f64 = F.dtype == SWALBE_F64;
+  LoopPlan L{{-1, 1, 0.0}, 0, false, false};
+  if (o->variant != 0 || o->tile_y > 0) return L;
+  L.multi = multi_shape(F.Lx, F.Ly, f64, sp.read_ft != 0, nsteps);
+  // larger films whose loop writes f and p on its last step only march in strips
+  if (final_only) L.march = march_segment(F.Lx, F.Ly, f64, sp.thermal != 0, nsteps, L.multi);
+  if (L.march > 0) L.multi.geom = -1;
+  L.single_tiles = f64 && L.multi.geom >= kTwoStepGeom;
+  L.last_tiles = f64 && L.march > 0;
+  return L;
+}
+
 // `multi`: nsub steps from t in one launch of its shape (geom >= 0).
 template <typename T>
 void enqueue_step(swalbe_state* st, const StepParams& sp, StepSeries ser, uint64_t t, int tile_y,
@@ -1024,15 +1047,9 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
   // launch of its own (its input moments stay in the other buffer for
   // materialize_last), and so is every step that something falls between:
   // a mass record or a measurement before step t, a snapshot after it.
-  const bool automatic = o->variant == 0 && o->tile_y <= 0;
-  MultiShape multi =
-      automatic ? multi_shape(F.Lx, F.Ly, F.dtype == SWALBE_F64, sp.read_ft != 0)
-                : MultiShape{-1, 1, 0.0};
-  // larger films whose loop writes f and p on its last step only march in strips
-  const int march = automatic && final_only ? march_segment(F.Lx, F.Ly, F.dtype == SWALBE_F64,
-                                                            sp.thermal != 0, multi)
-                                            : 0;
-  if (march > 0) multi.geom = -1;
+  const LoopPlan plan = loop_plan(F, sp, o, nsteps, final_only);
+  const MultiShape& multi = plan.multi;
+  const MultiShape one{-1, 1, 0.0};
   auto steps_at = [&](int64_t it) -> int64_t {
     if (multi.geom < 0 || want_meas) return 1;
     int64_t k = std::min<int64_t>(multi.k, nsteps - it);
@@ -1061,13 +1078,19 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
                       st->nparts, lb.meas + 4 * (it - 1), st->stream));
     }
     const StepSeries ser = series.at(it - 1);
-    const bool outs = multi.geom >= 0 ? it == nsteps : !final_only || it == nsteps;
+    const bool final_step = it == nsteps;
+    const bool tiles = final_step ? plan.single_tiles || plan.last_tiles
+                                  : plan.single_tiles && nsub == 1;
+    bool outs = multi.geom >= 0 ? final_step : !final_only || final_step;
+    if (tiles && sp.read_ft) outs = true;  // the next step reads them
+    const MultiShape& shape = tiles ? one : multi;
+    const int march = tiles ? 0 : plan.march;
     if (F.dtype == SWALBE_F64)
       enqueue_step<double>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
-                           multi, (int)nsub, march);
+                           shape, (int)nsub, march);
     else
       enqueue_step<float>(st, sp, ser, (uint64_t)t, tile_y, o->variant, o->nontemporal, outs,
-                           multi, (int)nsub, march);
+                          shape, (int)nsub, march);
     series.taken(it - 1, nsub, st->stream);
     if (want_snap && (t + nsub - 1) % o->snap_every == 0) {
       const int r = (int)(ksnap % SnapRing::R);
@@ -1135,6 +1158,25 @@ extern "C" {
 int swalbe_time_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps,
                      const swalbe_step_opts* opts) {
   return run_loop(st, p, nsteps, opts, nullptr);
+}
+
+int swalbe_loop_kernel(swalbe_state* st, const swalbe_params* p, int64_t nsteps,
+                       const swalbe_step_opts* o, int32_t out[4]) {
+  SW_CHECK_STATE(st);
+  if (!p || !out || nsteps < 0) {
+    set_error("swalbe_loop_kernel: null params or output, or negative step count");
+    return SWALBE_EINVAL;
+  }
+  if (int rc = set_device(st)) return rc;
+  swalbe_step_opts zero{};
+  if (!o) o = &zero;
+  const StepParams sp = make_step_params(p, o, 0);
+  const LoopPlan L = loop_plan(st->film, sp, o, nsteps, o->final_outputs_only && !sp.read_ft);
+  out[0] = L.multi.geom >= 0 ? 1 : L.march > 0 ? 2 : 0;
+  out[1] = L.multi.geom >= 0 ? L.multi.geom : L.march;
+  out[2] = L.multi.geom >= 0 ? L.multi.k : 1;
+  out[3] = L.single_tiles || L.last_tiles ? 1 : 0;
+  return SWALBE_OK;
 }
 
 int swalbe_time_loop_timed(swalbe_state* st, const swalbe_params* p, int64_t nsteps,

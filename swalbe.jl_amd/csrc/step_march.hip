@@ -15,10 +15,15 @@
 // the 64 x 16 LDS tiles, whose halo and per-population collisions cost 307;
 // FP64 206 against 287 us, with noise 320 against 409; 2500 x 2501 FP64 with
 // noise 124 against 161; 2000 x 1500 FP32 21 against 26, FP64 37 against 56.
-// A step that also writes f and p is the tiles' (196 against 290 us and more
-// at 4096 x 4096 FP32: a strip's 58 columns start on no line, nine times per
-// node), so this kernel writes them on a loop's last step only; τ ≠ 1, which
-// writes them on every step, stays with the tiles.  Two columns per lane (120
+// A step that also writes f and p is the tiles' (FP64 465 against 670 us at
+// 4096 x 4096, 90 against 108 at 2000 x 1500: a strip's 58 columns start on no
+// line, nine times per node), so an FP64 loop takes its last step there, with
+// the same bits, and τ ≠ 1, which writes them on every step, stays there.  An
+// FP32 loop takes every step here, for the same bits however a run is cut into
+// loops: its last step costs what the tiles' does wherever a row of the film
+// starts on no line either (2501 x 2499 142 against 135 us, 176 with the tiles'
+// streaming stores; 4100 x 4100 363 against 381) or the outputs fit the last
+// level cache (2000 x 1500 53 against 54).  Two columns per lane (120
 // written, on 32-byte sectors) were as fast at 4096 x 4096 (106, 204 us) and
 // slower on smaller films (2000 x 1500 FP32 23 us).
 #include <math.h>
@@ -115,11 +120,8 @@ struct March {
   __device__ __forceinline__ T get(const T* plane, int64_t row) const {
     return *(const GT*)(uniform(plane + row) + off);
   }
-  template <bool NT>
   __device__ __forceinline__ void put(T* plane, int64_t row, T v) const {
-    GT* q = (GT*)(const_cast<gbytes*>(uniform(plane + row)) + off);
-    if constexpr (NT) __builtin_nontemporal_store(v, q);
-    else *q = v;
+    *(GT*)(const_cast<gbytes*>(uniform(plane + row)) + off) = v;
   }
 
   __device__ __forceinline__ void prefetch(int j) {
@@ -308,13 +310,13 @@ struct March {
           vn = ih.div(my);
         }
         const int64_t r = (int64_t)R.Lx * j;
-        put<false>(io.h_out, r, s);
-        put<false>(io.ux_out, r, un);
-        put<false>(io.uy_out, r, vn);
+        put(io.h_out, r, s);
+        put(io.ux_out, r, un);
+        put(io.uy_out, r, vn);
         if constexpr (WF) {
 #pragma unroll
-          for (int k = 0; k < kQ; ++k) put<true>(io.f_out + k * R.fstride, r, g[k]);
-          put<true>(io.p_out, r, p0.v);
+          for (int k = 0; k < kQ; ++k) put(io.f_out + k * R.fstride, r, g[k]);
+          put(io.p_out, r, p0.v);
         }
       }
     }
@@ -397,17 +399,21 @@ void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
     if (sp.g != 0.0) SW_W(TH, WF, true);     \
     else SW_W(TH, WF, false);                \
   } while (0)
-  if (sp.thermal) {
-    if (write_f) SW_G(true, true);
-    else SW_G(true, false);
-  } else {
-    if (write_f) SW_G(false, true);
-    else SW_G(false, false);
+  if constexpr (sizeof(T) == 4) {
+    if (write_f) {
+      if (sp.thermal) SW_G(true, true);
+      else SW_G(false, true);
+      return;
+    }
   }
+  if (sp.thermal) SW_G(true, false);
+  else SW_G(false, false);
 #undef SW_G
 #undef SW_W
 #undef SW_S
 }
+
+constexpr int64_t kMarchShort = 16;
 
 // What a step costs: fixed + row us for each row that a wave computes (its
 // segment and `lead` of start-up), times the waves n that share a SIMD, or
@@ -432,11 +438,19 @@ constexpr MarchCost kMarchCost[2][2] = {{{3.5, 0.33, 1.0, 1.7}, {4.5, 0.42, 1.1,
 // 9.7, 850² 11.9 -> 9.9 / 13.0 -> 12.2, 1024² 11.9 -> 11.5 / 13.5 -> 15.0 (four
 // tiles on every CU), 4000 x 300 15.2 -> 12.1 / 17.1 -> 15.5.
 //
+// An FP32 film of 4 M nodes and more whose rows start on half a line writes f
+// and p in tiles in much less time (us, strips / tiles: 2048² 91 / 68, 16000 x
+// 1000 365 / 208, 4096² 368 / 206, 6000² 799 / 477), which a loop makes up for
+// after 3 to 16 steps without f and p (2048² 26.8 / 35.6, with noise 36.0 /
+// 39.0; 4096² 103 / 116, 123 / 132; 8192² 422 / 448, 442 / 510): loops of up
+// to kMarchShort steps stay with the tiles.
+//
 // Large FP64 films take four waves per SIMD while that gives segments of up to
 // 32 rows, and six beyond: 2500 x 2501 77 us with 28 rows (four), 82 with the
 // 18 of the model; 4096 x 4096 210 with 48 (six), 214 with 24.
-int march_segment(int Lx, int Ly, bool f64, bool noise, const MultiShape& other) {
+int march_segment(int Lx, int Ly, bool f64, bool noise, int64_t nsteps, const MultiShape& other) {
   if (Lx < 64 || Ly < 8) return 0;
+  if (!f64 && nsteps <= kMarchShort && Lx % 16 == 0 && (int64_t)Lx * Ly >= 4000000) return 0;
   const int64_t cus = device_cus(), simds = 4 * cus;
   const int64_t strips = (Lx - 1) / kMarchOut + 1, rows = strips * Ly;
   const int64_t four = (rows - 1) / (4 * simds) + 1, six = (rows - 1) / (6 * simds) + 1;

@@ -427,7 +427,7 @@ struct Geom {
   double fixed, body;
   int wgs;
 };
-constexpr int kNGeoms = 5;
+constexpr int kNGeoms = 5;  // those from kTwoStepGeom on have k = 2
 constexpr Geom kGeoms64[kNGeoms] = {{8, 8, 3, 3.6, 3.2, 1},
                                     {16, 16, 3, 2.0, 7.5, 1},
                                     {24, 16, 2, 2.6, 5.9, 1},
@@ -485,7 +485,7 @@ void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uin
 // FP64 64² 2.32 / 7.48, 256² 3.14 / 7.35, 512² 7.92 / 8.94, 700 x 640 13.9 /
 // 12.7; FP32 64² 2.01 / 8.06, 256² 2.34 / 8.10, 512² 5.32 / 9.04, 850² 11.2 /
 // 11.6, 1024² 14.2 / 11.9.
-MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried) {
+MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried, int64_t nsteps) {
   const int64_t cus = device_cus();
   auto rounds = [&](int tx, int ty, int wgs) {
     const int64_t tiles = (int64_t)((Lx - 1) / tx + 1) * ((Ly - 1) / ty + 1);
@@ -493,6 +493,10 @@ MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried) {
   };
   const double r = rounds(64, f64 ? 8 : 16, 1);
   double least = f64 ? 5.0 + 2.1 * r : r <= 4.0 ? 7.6 + 1.05 * r : 6.0 + 1.85 * r;
+  // FP64 with τ ≠ 1: the halo's populations weigh more than the model's.  us per
+  // step, one / several steps: 900 x 700 34.8 / 35.3, with noise 38.5 / 44.6;
+  // 560² 21.0 / 20.4, 24.9 / 25.9; 500² (modelled at 0.85) 17.7 / 14.0, 21.0 / 18.0.
+  if (carried && f64) least *= 0.9;
   MultiShape best{-1, 1, least};
   for (int i = 0; i < kNGeoms; ++i) {
     const Geom& g = f64 ? kGeoms64[i] : kGeoms32[i];
@@ -507,8 +511,17 @@ MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried) {
   // / two steps: 1000 x 1031 24.5 / 23.8, 1200² 32.7 / 33.5, 1300 x 1250 44.5 /
   // 35.8, 2000 x 1500 78 / 64, 3000² 256 / 180, 4096² 389 / 323, with noise 397
   // / 355.  FP64 tiles are bound by arithmetic: 2000 x 1500 118 / 141.
-  if (carried && !f64 && best.geom < 0 && (int64_t)Lx * Ly >= 1600000)
-    best = MultiShape{3, kGeoms32[3].k, least};
+  // A launch of one of its two steps, which every loop ends with and a loop of
+  // an even number takes twice, costs more than the one-step kernel's (us per
+  // loop of one step, one / two: 750² 37 / 40, 1300 x 1250 62 / 76, 4096² 430 /
+  // 610), and FP32 bits must not depend on where a launch falls, so short loops
+  // stay with the one-step kernel (us per step of loops of 3 steps: 750² 26.3 /
+  // 23.5, 4096² with noise 407 / 428).
+  if (carried && !f64) {
+    const bool large = best.geom < 0 && (int64_t)Lx * Ly >= 1600000;
+    if (large) best = MultiShape{3, kGeoms32[3].k, least};
+    if (best.geom >= kTwoStepGeom && nsteps < (large ? 9 : 4)) best = MultiShape{-1, 1, least};
+  }
   return best;
 }
 

@@ -267,17 +267,18 @@ struct MultiShape {
   int k;
   double us;  // the path's modelled time per step without noise
 };
-MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried);
+constexpr int kTwoStepGeom = 2;  // the shapes from here on take two steps per launch
+MultiShape multi_shape(int Lx, int Ly, bool f64, bool carried, int64_t nsteps);
 template <typename T>
 void launch_multi(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step, int k,
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int geom,
                   hipStream_t s);
 
 // One τ = 1 step of a larger film, a wave per strip of columns and segment of
-// `seg` rows (step_march.hip), writing the moments, and f and p with write_f.
-// march_segment: the rows per segment for a film, 0 where `other` (the path
-// multi_shape chose) is faster.
-int march_segment(int Lx, int Ly, bool f64, bool noise, const MultiShape& other);
+// `seg` rows (step_march.hip), writing the moments, and f and p with write_f
+// (FP32 only).  march_segment: the rows per segment for a loop of nsteps steps
+// of a film, 0 where `other` (the path multi_shape chose) is faster.
+int march_segment(int Lx, int Ly, bool f64, bool noise, int64_t nsteps, const MultiShape& other);
 template <typename T>
 void launch_march(const StepIO<T>& io, const StepParams& sp, StepSeries ser, uint64_t step,
                   bool write_f, int Lx, int Ly, int64_t fstride, Enc enc, int seg, hipStream_t s);

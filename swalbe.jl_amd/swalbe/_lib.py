@@ -143,6 +143,8 @@ def lib():
     _sig(L, "swalbe_step_forces", [_V, C.POINTER(Params), _I, C.c_uint64, C.c_uint64])
     _sig(L, "swalbe_step_advance", [_V, _D, _D])
     _sig(L, "swalbe_time_loop", [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts)])
+    _sig(L, "swalbe_loop_kernel", [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts),
+                                   C.POINTER(_I)])
     _sig(L, "swalbe_time_loop_timed",
          [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts), C.POINTER(_D)])
     _sig(L, "swalbe_reduce", [_V, _I, _D, C.POINTER(_D)])

@@ -641,7 +641,7 @@ def time_loop(sys: SysConst, state: HipState, *args, verbose: bool = False, ther
     o.variant = int(variant)  # FP32 kernel: 0 default, 1 / 2 LDS tiles, 3 strips
     final_outputs_only = P.τ == 1.0 and (bool(final_outputs_only) or (tile_y == 0 and variant == 0))
     o.nontemporal = int(nontemporal) if nontemporal is not None else store_mode(
-        sys.Lx, sys.Ly, state.T is np.float64, final_outputs_only)
+        sys.Lx, sys.Ly, state.T is np.float64, final_outputs_only and nsteps > 1)
     keep = []
     dh = None
     f = measure = None
