@@ -38,23 +38,26 @@ inline int copy_threads(size_t bytes) {
 }
 
 // ---------------------------------------------------------------- pinned buffers
+constexpr int kFlags = 16;
+
 struct Stage {
   int device = 0;
-  char* pin = nullptr;  // kChunk bytes and the flag behind them
+  char* pin = nullptr;  // kChunk bytes and the flags behind them
   hipEvent_t ev = nullptr;
-  uint32_t seq = 0;  // the flag's value after the buffer's last flagged kernel
+  uint32_t seq = 0;  // the flags' value after the buffer's last flagged kernel
 
   uint32_t* flag() const { return (uint32_t*)(pin + kChunk); }
 };
 
-// Waits for a kernel that ends by setting its buffer's flag: polls for up to
-// 100 us, which is quicker by 5 us than waiting for the stream, then waits for
-// the stream (which also reports a kernel that failed).
-hipError_t flag_wait(const Stage& st, hipStream_t s) {
+// Waits for a kernel whose n workgroups end by setting a flag of its buffer
+// each: polls for up to 100 us, which is quicker by 5 us than waiting for the
+// stream, then waits for the stream (which also reports a kernel that failed).
+hipError_t flag_wait(const Stage& st, int n, hipStream_t s) {
   const auto t0 = std::chrono::steady_clock::now();
   for (;;) {
     for (int i = 0; i < 64; ++i) {
-      if (__atomic_load_n(st.flag(), __ATOMIC_ACQUIRE) == st.seq) return hipSuccess;
+      while (n > 0 && __atomic_load_n(st.flag() + n - 1, __ATOMIC_ACQUIRE) == st.seq) --n;
+      if (n == 0) return hipSuccess;
       __builtin_ia32_pause();
     }
     if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(100))
@@ -93,9 +96,9 @@ hipError_t stage_take(int device, Stage* out) {
   }
   Stage s;
   s.device = device;
-  hipError_t e = hipHostMalloc((void**)&s.pin, kChunk + 64,
+  hipError_t e = hipHostMalloc((void**)&s.pin, kChunk + kFlags * sizeof(uint32_t),
                                hipHostMallocPortable | hipHostMallocCoherent);
-  if (e == hipSuccess) *s.flag() = 0;
+  for (int i = 0; e == hipSuccess && i < kFlags; ++i) s.flag()[i] = 0;
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s.ev, hipEventDisableTiming);
   if (e != hipSuccess) {
     stage_free(s);
@@ -183,11 +186,13 @@ __global__ __launch_bounds__(256) void k_reencode(float* __restrict__ dev, int64
   }
 }
 
-// A small field in one workgroup, which tells the host by a flag behind the
-// data.  A download of 1024 doubles takes 9.9 us instead of 15.2 with a wait for
-// the stream, an upload 10.8 instead of 16; at 4096 12 and 15, at 8192 one
-// workgroup is no faster.
-constexpr int64_t kSmall = 4096;  // elements
+// A small field in a few workgroups, each of which tells the host by a flag
+// behind its data.  us, with a wait for the stream / so: doubles 1000 down 14 / 9,
+// 8000 down 14.8 / 11.3 (the runtime's copy of pageable memory 12) and up 14.8 /
+// 10.8 (11.2), 65536 down 32 / 30 and up 29 / 25.  Four elements a thread one after
+// the other took 13.5 for 8000 up, one workgroup more than the stream.
+constexpr int64_t kSmall = 1024;  // elements of a workgroup, while there are flags for it
+constexpr int64_t kFlagged = 65536;
 
 template <typename TD, typename TH, bool BITS, bool DOWN>
 __global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __restrict__ pin,
@@ -195,7 +200,8 @@ __global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __rest
                                                 Offsets off, uint32_t* flag, uint32_t seq) {
   for (int k = 0; k < planes; ++k) {
     const double o = off.v[k];
-    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+#pragma unroll 4
+    for (int64_t i = blockIdx.x * 1024 + threadIdx.x; i < n; i += 1024 * (int64_t)gridDim.x) {
       if constexpr (BITS) {
         if constexpr (DOWN) pin[k * n + i] = dev[k * stride + i];
         else dev[k * stride + i] = pin[k * n + i];
@@ -207,12 +213,15 @@ __global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __rest
       }
     }
   }
-  // every wave's stores have left before the flag's release, which writes the
-  // L2 back for all of them (a fence at workgroup scope waits for none)
+  // a download: every wave's stores have left before the flag's release, which
+  // writes the L2 back for all of them (a fence at workgroup scope waits for
+  // none); an upload: its loads are back, and the stream orders the plane's next
+  // use behind this kernel
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
-    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(flag + blockIdx.x, seq, DOWN ? __ATOMIC_RELEASE : __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 Offsets offsets(const double* off, int planes) {
@@ -231,8 +240,12 @@ struct Job {
   int planes, device;
   Offsets off;
   bool bits;
-  bool small;   // one workgroup and a flag (k_small)
+  int groups;   // > 0: so many workgroups, each with a flag (k_small)
   bool single;  // one chunk: its end is the stream's, no event (0.9 us less of 16)
+  // an FP32 film and doubles: converted on the host, which crosses half the
+  // bytes (200000 doubles up 80 -> 50 us, 1e6 down 270 -> 189); not one so small
+  // that a single workgroup takes it
+  bool narrow;
   hipStream_t s;
   std::atomic<int64_t> next{0};
   std::atomic<int> err{0};
@@ -242,10 +255,10 @@ struct Job {
 template <typename TD, typename TH, bool BITS>
 void launch_small(const Job& J, const Stage& st) {
   if (J.down)
-    hipLaunchKernelGGL((k_small<TD, TH, BITS, true>), dim3(1), dim3(1024), 0, J.s, (TD*)J.dev,
+    hipLaunchKernelGGL((k_small<TD, TH, BITS, true>), dim3(J.groups), dim3(1024), 0, J.s, (TD*)J.dev,
                        (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
   else
-    hipLaunchKernelGGL((k_small<TD, TH, BITS, false>), dim3(1), dim3(1024), 0, J.s, (TD*)J.dev,
+    hipLaunchKernelGGL((k_small<TD, TH, BITS, false>), dim3(J.groups), dim3(1024), 0, J.s, (TD*)J.dev,
                        (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
 }
 
@@ -278,11 +291,13 @@ hipError_t issue(const Job& J, Stage& st, int64_t a, int64_t b) {
   Piece P{a, b, J.n, J.stride, (int)(a / J.n)};
   const int64_t widest = b - a < J.n ? b - a : J.n;
   const dim3 grid((unsigned)((widest + 255) / 256), (unsigned)((b - 1) / J.n - a / J.n + 1));
-  if (J.small) ++st.seq;
+  if (J.groups) ++st.seq;
   with_types(J, [&](auto td, auto th, auto bits) {
     using TD = decltype(td);
     using TH = decltype(th);
-    if (J.small) launch_small<TD, TH, decltype(bits)::value>(J, st);
+    if (J.groups && J.narrow) launch_small<uint32_t, uint32_t, true>(J, st);
+    else if (J.groups) launch_small<TD, TH, decltype(bits)::value>(J, st);
+    else if (J.narrow) launch_piece<uint32_t, uint32_t, true>(J, st.pin, P, grid);
     else launch_piece<TD, TH, decltype(bits)::value>(J, st.pin, P, grid);
   });
   hipError_t e = hipGetLastError();
@@ -309,6 +324,15 @@ void convert(const Job& J, TD* t, int64_t a, int64_t b) {
   }
 }
 
+// Elements [a, b) between the host array and a pinned buffer
+void stage_copy(const Job& J, char* pin, int64_t a, int64_t b) {
+  char* const h = J.host + (size_t)a * J.hes;
+  const size_t bytes = (size_t)(b - a) * J.hes;
+  if (J.narrow) convert<float, double>(J, (float*)pin, a, b);
+  else if (J.down) memcpy(h, pin, bytes);
+  else memcpy(pin, h, bytes);
+}
+
 // One copying thread: claims chunks until none is left, two buffers in turn
 // (the GPU fills or drains one while the host copies the other).
 void run_chunks(Job* pJ) {
@@ -318,11 +342,11 @@ void run_chunks(Job* pJ) {
   hipError_t e = hipSetDevice(J.device);
   auto finish = [&](int r) {  // wait for buffer r; a download's chunk goes to the caller
     if (b[r] < 0) return;
-    const hipError_t w = J.small    ? flag_wait(st[r], J.s)
+    const hipError_t w = J.groups   ? flag_wait(st[r], J.groups, J.s)
                          : J.single ? hipStreamSynchronize(J.s)
                                     : hipEventSynchronize(st[r].ev);
     if (w == hipSuccess && J.down && e == hipSuccess)
-      memcpy(J.host + (size_t)a[r] * J.hes, st[r].pin, (size_t)(b[r] - a[r]) * J.hes);
+      stage_copy(J, st[r].pin, a[r], b[r]);
     if (e == hipSuccess) e = w;
     b[r] = -1;
   };
@@ -340,8 +364,7 @@ void run_chunks(Job* pJ) {
     if (e != hipSuccess) break;
     a[r] = c * J.per;
     const int64_t end = a[r] + J.per < J.total ? a[r] + J.per : J.total;
-    if (!J.down)
-      memcpy(st[r].pin, J.host + (size_t)a[r] * J.hes, (size_t)(end - a[r]) * J.hes);
+    if (!J.down) stage_copy(J, st[r].pin, a[r], end);
     e = issue(J, st[r], a[r], end);
     if (e == hipSuccess) b[r] = end;
   }
@@ -394,9 +417,10 @@ int transfer(bool down, void* host, size_t hes, void* dev, size_t des, int64_t n
   J.stride = stride;
   J.planes = planes;
   J.total = n * planes;
-  J.per = (int64_t)(kChunk / hes);
+  J.groups = J.total > kFlagged ? 0 : J.total > kFlags * kSmall ? kFlags : (int)((J.total - 1) / kSmall + 1);
+  J.narrow = J.groups != 1 && des < hes;
+  J.per = (int64_t)(kChunk / (J.narrow ? des : hes));
   J.single = J.total <= J.per;
-  J.small = J.total <= kSmall;
   J.device = device;
   J.off = offsets(off, planes);
   J.bits = hes == des;
@@ -458,7 +482,7 @@ uint32_t* HostResult::flag() const { return p_ ? ((Stage*)stage_)->flag() : null
 uint32_t HostResult::seq() { return p_ ? ++((Stage*)stage_)->seq : 0; }
 
 hipError_t HostResult::get(double* out, int n) {
-  const hipError_t e = p_ ? flag_wait(*(Stage*)stage_, s_) : hipStreamSynchronize(s_);
+  const hipError_t e = p_ ? flag_wait(*(Stage*)stage_, 1, s_) : hipStreamSynchronize(s_);
   if (e == hipSuccess && p_) memcpy(out, p_, sizeof(double) * (size_t)n);
   return e;
 }
