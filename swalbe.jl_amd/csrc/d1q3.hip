@@ -438,9 +438,13 @@ __global__ __launch_bounds__(NB) void k1_step(Film1 S, uint64_t step, swalbe::St
   }
 }
 
-// a / d, correctly rounded
-__device__ __forceinline__ double quotient(double a, double d) { return swalbe::Recip(d).div(a); }
+// a / d, correctly rounded (_normal: a not near the subnormals)
+__device__ __forceinline__ double quotient(double a, double d) { return swalbe::Recip<>(d).div(a); }
+__device__ __forceinline__ double quotient_normal(double a, double d) {
+  return swalbe::Recip<false>(d).div(a);
+}
 __device__ __forceinline__ float quotient(float a, float d) { return a / d; }
+__device__ __forceinline__ float quotient_normal(float a, float d) { return a / d; }
 
 // Pointers read from the film table are generic to the compiler, which then
 // emits flat loads and stores (they wait on the LDS counter as well).  All of
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(64) void k1_wave(Film1 S, uint64_t step0, int k, in
         for (int j = 0; j < NPT; ++j) {
           const T hm = j > 0 ? h[j > 0 ? j - 1 : 0] : hl;
           const T hp = j < NPT - 1 ? h[j < NPT - 1 ? j + 1 : 0] : hr;
-          const T a = quotient(hmin, h[j] + hcrit);
+          const T a = quotient_normal(hmin, h[j] + hcrit);
           const T v = -gam[j] * (kap[j] * disjoin_law(a, usual ? 9 : n, usual ? 3 : m));
           p[j] = v - gam[j] * ((hm - T(2) * h[j]) + hp);
         }

@@ -145,7 +145,7 @@ struct March {
       const T L = (T(2.0 / 3.0) * (((hjp + hip) + him) + hjm) +
                    T(1.0 / 6.0) * (((hipjp + himjp) + himjm) + hipjm)) -
                   T(10.0 / 3.0) * h;
-      const T q = Recip(h + sp.hcrit).div(sp.hmin);
+      const T q = Recip<false>(h + sp.hcrit).div(sp.hmin);
       const T p0 = -sp.gamma * (kap * powlaw(q, sp.n, sp.m, sp.powmode));
       return p0 - sp.gamma * L;
     }
@@ -214,7 +214,7 @@ struct March {
       const T gy = T(-1.0 / 3.0) * (fjp - fjm) -
                    T(1.0 / 12.0) * (((fipjp + fimjp) - fimjm) - fipjm);
       const T hgx = h * gx, hgy = h * gy;
-      const Recip iden((T(2) * (h * h) + sp.c6d * h) + sp.c3dd);
+      const Recip<> iden((T(2) * (h * h) + sp.c6d * h) + sp.c3dd);
       const T sx = iden.div(sp.c6mu * h * u);
       const T sy = iden.div(sp.c6mu * h * v);
       T Fx = -hgx - sx;
@@ -222,7 +222,7 @@ struct March {
       if constexpr (TH) {
         double z0, z1;
         box_muller(u32(wa), u32(wb), &z0, &z1);
-        const T amp = sqrt(Recip(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
+        const T amp = sqrt(Recip<false>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
                                .div(sp.kb26 * h));
         Fx = Fx - z0 * amp;
         Fy = Fy - z1 * amp;
@@ -305,7 +305,7 @@ struct March {
           un = mx * ih;
           vn = my * ih;
         } else {
-          const Recip ih(s);
+          const Recip<> ih(s);
           un = ih.div(mx);
           vn = ih.div(my);
         }

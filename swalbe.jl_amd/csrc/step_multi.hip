@@ -196,7 +196,7 @@ struct Multi {
                      T(1.0 / 6.0) * (((hipjp + himjp) + himjm) + hipjm)) -
                     T(10.0 / 3.0) * h;
         const T kap = io.kappa ? plane(kK)[o] : (T)sp.kappa;
-        const T a = Recip(h + sp.hcrit).div(sp.hmin);
+        const T a = Recip<false>(h + sp.hcrit).div(sp.hmin);
         const T p0 = -sp.gamma * (kap * powlaw(a, sp.n, sp.m, sp.powmode));
         p = p0 - sp.gamma * L;
       }
@@ -293,7 +293,7 @@ struct Multi {
         const T gy = T(-1.0 / 3.0) * (fjp - fjm) -
                      T(1.0 / 12.0) * (((fipjp + fimjp) - fimjm) - fipjm);
         const T hgx = h * gx, hgy = h * gy;
-        const Recip iden((T(2) * (h * h) + sp.c6d * h) + sp.c3dd);
+        const Recip<> iden((T(2) * (h * h) + sp.c6d * h) + sp.c3dd);
         const T sx = iden.div(sp.c6mu * h * u);
         const T sy = iden.div(sp.c6mu * h * v);
         T Fx = -hgx - sx;
@@ -301,7 +301,7 @@ struct Multi {
         if constexpr (TH) {
           double z0, z1;
           normal_pair(sp.seed, step, ni, kTagThermal, &z0, &z1);
-          const T amp = sqrt(Recip(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
+          const T amp = sqrt(Recip<false>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
                                  .div(sp.kb26 * h));
           Fx = Fx - z0 * amp;
           Fy = Fy - z1 * amp;
@@ -315,7 +315,8 @@ struct Multi {
 #pragma unroll
         for (int k = 0; k < kQ; ++k) {
           T f;
-          if constexpr (GRAV) f = feq_k<T>(k, h, u, v, usq, c56g, g0);
+          // (k = 0: NaN for an infinite height, as the force makes the others)
+          if (GRAV || k == 0) f = feq_k<T>(k, h, u, v, usq, c56g, g0);
           else f = feq_k0<T>(k, h, u, v, usq);
           if constexpr (RFT) f = sp.omeg * F[k * RN] + sp.itau * f;
           F[k * RN] = k > 0 ? f + force_term<T>(k, Fx, Fy) : f;
@@ -348,7 +349,7 @@ struct Multi {
         u[q] = mx * ih;
         v[q] = my * ih;
       } else {
-        const Recip ih(sum);
+        const Recip<> ih(sum);
         u[q] = ih.div(mx);
         v[q] = ih.div(my);
       }

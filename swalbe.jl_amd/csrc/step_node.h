@@ -32,23 +32,30 @@ __device__ __forceinline__ T powlaw(T a, int n, int m, int mode) {
   return tn - tm;
 }
 
-// 1 / d refined to the point where a quotient by d takes three more
-// operations: the instruction sequence of an IEEE FP64 division (v_rcp_f64,
-// two Newton steps, quotient, residual correction: Markstein, IBM J. Res. Dev.
-// 34 (1990) 111) without the operand scaling, so the quotient is the correctly
-// rounded a / d, the compiler's bits, wherever d, a and a / d lie within
-// 2^±900; zero, infinite and NaN operands go through v_div_fixup as in the
-// compiler's sequence.  Several quotients by one d share the first five
-// operations.
+// 1 / d refined to the point where a quotient by d takes three more operations:
+// the instruction sequence of an IEEE FP64 division (v_rcp_f64, two Newton
+// steps, quotient, residual correction: Markstein, IBM J. Res. Dev. 34 (1990)
+// 111) without the scaling by cases.  Instead both operands are taken 2^64 times
+// as large (S), so that the residual a - d q is exact down to subnormal a and the
+// quotient the correctly rounded a / d, the compiler's bits, wherever a and d lie
+// below 2^950 and d above 2^-12 (a subnormal quotient that lies halfway between
+// two excepted).  Velocities do become that small: ahead of a front they halve
+// with about every node, and 3 in 100 subnormal quotients come out wrong without.
+// Zero, infinite and NaN operands go through v_div_fixup as in the compiler's
+// sequence; operands beyond 2^950 count as infinite.  Several quotients by one d
+// share the first six operations.  S costs two operations for a d and one quotient
+// (0 to 3 % of a step, 4 of a line's of 3e6 nodes); a numerator that is a parameter
+// of the film does without.
+template <bool S = true>
 struct Recip {
   double d, r;
-  __device__ __forceinline__ explicit Recip(double den) : d(den) {
-    double x = __builtin_amdgcn_rcp(den);
-    x = __builtin_fma(__builtin_fma(-den, x, 1.0), x, x);
-    r = __builtin_fma(__builtin_fma(-den, x, 1.0), x, x);
+  __device__ __forceinline__ explicit Recip(double den) : d(S ? den * 0x1p64 : den) {
+    double x = __builtin_amdgcn_rcp(d);
+    x = __builtin_fma(__builtin_fma(-d, x, 1.0), x, x);
+    r = __builtin_fma(__builtin_fma(-d, x, 1.0), x, x);
   }
-  __device__ __forceinline__ double div(double a) const {
-    const double q = a * r;
+  __device__ __forceinline__ double div(double num) const {
+    const double a = S ? num * 0x1p64 : num, q = a * r;
     return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, a), r, q), d, a);
   }
 };
