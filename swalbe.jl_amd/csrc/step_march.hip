@@ -222,7 +222,7 @@ struct March {
       if constexpr (TH) {
         double z0, z1;
         box_muller(u32(wa), u32(wb), &z0, &z1);
-        const T amp = sqrt(Recip<false>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
+        const T amp = sqrt(Recip<>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
                                .div(sp.kb26 * h));
         Fx = Fx - z0 * amp;
         Fy = Fy - z1 * amp;

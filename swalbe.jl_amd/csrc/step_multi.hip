@@ -301,7 +301,7 @@ struct Multi {
         if constexpr (TH) {
           double z0, z1;
           normal_pair(sp.seed, step, ni, kTagThermal, &z0, &z1);
-          const T amp = sqrt(Recip<false>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
+          const T amp = sqrt(Recip<>(((T(2) * h) * h + (T(6) * h) * sp.delta) + sp.d3dd)
                                  .div(sp.kb26 * h));
           Fx = Fx - z0 * amp;
           Fy = Fy - z1 * amp;
