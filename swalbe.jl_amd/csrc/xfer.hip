@@ -194,14 +194,16 @@ __global__ __launch_bounds__(256) void k_reencode(float* __restrict__ dev, int64
 constexpr int64_t kSmall = 1024;  // elements of a workgroup, while there are flags for it
 constexpr int64_t kFlagged = 65536;
 
-template <typename TD, typename TH, bool BITS, bool DOWN>
+// ONE: at most one element of a plane for each thread (the loop's code alone
+// costs a small transfer 0.6 us)
+template <typename TD, typename TH, bool BITS, bool DOWN, bool ONE>
 __global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __restrict__ pin,
                                                 int planes, int64_t n, int64_t stride,
                                                 Offsets off, uint32_t* flag, uint32_t seq) {
+  const int64_t first = blockIdx.x * 1024 + threadIdx.x, step = 1024 * (int64_t)gridDim.x;
   for (int k = 0; k < planes; ++k) {
     const double o = off.v[k];
-#pragma unroll 4
-    for (int64_t i = blockIdx.x * 1024 + threadIdx.x; i < n; i += 1024 * (int64_t)gridDim.x) {
+    auto cross = [&](int64_t i) {
       if constexpr (BITS) {
         if constexpr (DOWN) pin[k * n + i] = dev[k * stride + i];
         else dev[k * stride + i] = pin[k * n + i];
@@ -211,6 +213,12 @@ __global__ __launch_bounds__(1024) void k_small(TD* __restrict__ dev, TH* __rest
       } else {
         dev[k * stride + i] = (TD)((double)pin[k * n + i] - o);
       }
+    };
+    if constexpr (ONE) {
+      if (first < n) cross(first);
+    } else {
+#pragma unroll 4
+      for (int64_t i = first; i < n; i += step) cross(i);
     }
   }
   // a download: every wave's stores have left before the flag's release, which
@@ -254,12 +262,14 @@ struct Job {
 
 template <typename TD, typename TH, bool BITS>
 void launch_small(const Job& J, const Stage& st) {
-  if (J.down)
-    hipLaunchKernelGGL((k_small<TD, TH, BITS, true>), dim3(J.groups), dim3(1024), 0, J.s, (TD*)J.dev,
-                       (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
-  else
-    hipLaunchKernelGGL((k_small<TD, TH, BITS, false>), dim3(J.groups), dim3(1024), 0, J.s, (TD*)J.dev,
-                       (TH*)st.pin, J.planes, J.n, J.stride, J.off, st.flag(), st.seq);
+  auto go = [&](auto down, auto one) {
+    hipLaunchKernelGGL((k_small<TD, TH, BITS, decltype(down)::value, decltype(one)::value>),
+                       dim3(J.groups), dim3(1024), 0, J.s, (TD*)J.dev, (TH*)st.pin, J.planes, J.n,
+                       J.stride, J.off, st.flag(), st.seq);
+  };
+  const bool one = J.n <= 1024 * (int64_t)J.groups;
+  if (J.down) one ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  else one ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 template <typename TD, typename TH, bool BITS>
