@@ -495,7 +495,7 @@ __device__ __forceinline__ T from_above(T v) {
 // steps.  Measured against the kernels it replaces for single films (us per
 // step): L = 1024 4.6 in one workgroup's LDS -> 0.47, over up to 256 CUs
 // instead of one; L = 3e6 36.4 with one launch and 64 bytes per node and step
-// -> 9.2, with 5 bytes per node and step.
+// -> 10.2, with 5 bytes per node and step.
 // The loop exists twice: for the usual law, n = 9, m = 3 and g = 0, without a
 // branch per node, so that the division chains of a lane's nodes overlap, and
 // for any other (one copy with the branches and the compiler's division: 0.51
@@ -1676,6 +1676,7 @@ hipError_t launch_resident(const Film1* d_table, int nfilms, int64_t nsteps, int
 // 65000 nodes up.  us per step: 1024 nodes (1, 10) 0.47, (2, 16) 0.53; 20000
 // (2, 16) 0.55, (1, 6) 0.69; 2e5 (4, 10) 1.05, (2, 10) 1.31; 1e6 (4, 10) 3.6,
 // (8, 24) 3.8; 3e6 (8, 10) 9.2, (4, 4) 9.8; 4e6 (8, 10) 11.8, (4, 4) 13.0.
+// (Before the divisions scaled their operands, which added 0 to 4 % to each.)
 struct WaveShape {
   int npt, k;
 };

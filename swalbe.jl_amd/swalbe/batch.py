@@ -4,7 +4,8 @@ Each film keeps its own parameters, size and step budget; every
 Batch.step(n) advances all resident films in one launch per time step.
 add/remove/step only enqueue work; get() waits for the film's own last step.
 A film's result is bit-identical to the same film stepped alone by
-time_loop on an FP32 HipState (both run the same tile kernel).
+time_loop on an FP32 HipState in the same tile kernel (variant=2 and a
+tile_y of 8 or 16); time_loop's default kernels agree to FP32 rounding.
 """
 from __future__ import annotations
 
