@@ -21,6 +21,7 @@ struct swalbe_state {
   double* partials = nullptr;  // reduction scratch, 4 doubles per block
   int nparts = 0;
   double* red_out = nullptr;   // 4 doubles
+  swalbe::SeriesBuf series;    // per-step series of short loops
 };
 
 namespace swalbe {
@@ -309,7 +310,7 @@ int swalbe_destroy(swalbe_state* st) {
   void* ptrs[] = {F.f[0],  F.f[1],  F.feq,   F.hbuf[0], F.hbuf[1], F.uxbuf[0], F.uxbuf[1],
                   F.uybuf[0], F.uybuf[1], F.vsq, F.pressure, F.Fx, F.Fy, F.slipx, F.slipy,
                   F.hgpx,  F.hgpy,  F.kbtx,  F.kbty,    F.theta,   F.kappa, st->partials,
-                  st->red_out};
+                  st->red_out, st->series.mem};
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (st->own_stream) hipStreamDestroy(st->own_stream);
@@ -998,7 +999,7 @@ int run_loop(swalbe_state* st, const swalbe_params* p, int64_t nsteps, const swa
   if (want_fluid) SW_HIP(hipMalloc((void**)&lb.fluid, (size_t)F.N * std::max<int64_t>(1, nsteps)));
   const double meas_thresh = o->surf_thresh > 0.0 ? o->surf_thresh : 0.055;
   SeriesRun series;
-  SW_HIP(series.start(nsteps, want_dh, want_wet, st->stream));
+  SW_HIP(series.start(nsteps, want_dh, want_wet, &st->series, st->stream));
   int64_t nmass = 0;
   for (int64_t it = 1; it <= nsteps && want_mass; ++it)
     if ((o->t0 + it) % p->tdump == 0) ++nmass;

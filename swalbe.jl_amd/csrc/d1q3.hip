@@ -1034,6 +1034,7 @@ struct swalbe_film1d {
   // film table of the ensembles this film was listed first in
   Film1* table = nullptr;
   int table_films = 0;
+  swalbe::SeriesBuf series;  // per-step series of short loops
 };
 
 namespace {
@@ -1335,7 +1336,7 @@ int swalbe1d_destroy(swalbe_film1d* s) {
   // with other films: this waits for theirs too)
   if (e == hipSuccess && s->stream) e = hipStreamSynchronize(s->stream);
   void* ptrs[] = {s->slab, s->theta, s->kap, s->gamma, s->grad_gamma, s->border[0],
-                  s->border[1], s->interior, s->table};
+                  s->border[1], s->interior, s->table, s->series.mem};
   for (void* p : ptrs)
     if (p) {
       const hipError_t ef = hipFree(p);
@@ -1753,7 +1754,7 @@ int loop_per_step(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
   const int64_t nmass = o->mass_series ? count_every(o->t0, nsteps, p->tdump) : 0;
   const int64_t nsnap = o->snap_series ? count_every(o->t0, nsteps, o->snap_every) : 0;
   bool ok = true;
-  ok = series.start(nsteps, o->dh_series, o->wet_series, s->stream) == hipSuccess;
+  ok = series.start(nsteps, o->dh_series, o->wet_series, &s->series, s->stream) == hipSuccess;
   if (nmass) ok = ok && hipMalloc(&mass, 32 * nmass) == hipSuccess;
   if (nsnap) ok = ok && hipMalloc(&snap, (size_t)nsnap * s->L * s->esz) == hipSuccess;
   hipError_t e = hipSuccess;

@@ -623,21 +623,33 @@ void launch_reduce_finish(const double* partials, int nparts, double* out, hipSt
 }
 
 SeriesRun::~SeriesRun() {
-  if (slots) (void)hipFree(slots);
-  if (folded) (void)hipFree(folded);
+  if (own) (void)hipFree(own);
 }
 
-hipError_t SeriesRun::start(int64_t n, bool want_dh, bool want_wet, hipStream_t s) {
+hipError_t SeriesRun::start(int64_t n, bool want_dh, bool want_wet, SeriesBuf* buf,
+                            hipStream_t s) {
   nsteps = n;
   dh = want_dh;
   wet = want_wet;
   if (n < 1 || (!want_dh && !want_wet)) return hipSuccess;
-  const int64_t held = n < kSeriesChunk ? n : kSeriesChunk;
-  hipError_t e = hipMalloc((void**)&slots, sizeof(unsigned long long) * held * kSeriesSlots *
-                                               kSeriesWords);
-  if (e != hipSuccess) slots = nullptr;
-  if (e == hipSuccess) e = hipMalloc((void**)&folded, sizeof(double) * 3 * n);
-  if (e != hipSuccess) return e;
+  const bool kept = n <= kSeriesKeep;
+  const int64_t held = kept ? kSeriesKeep : n < kSeriesChunk ? n : kSeriesChunk;
+  const size_t slot_bytes = sizeof(unsigned long long) * held * kSeriesSlots * kSeriesWords;
+  void* mem = kept ? buf->mem : nullptr;
+  if (!mem) {
+    const hipError_t e = hipMalloc(&mem, slot_bytes + sizeof(double) * 3 * (kept ? held : n));
+    if (e != hipSuccess) return e;
+    if (kept) *buf = SeriesBuf{mem, false};
+    else own = mem;
+  }
+  slots = (unsigned long long*)mem;
+  folded = (double*)((char*)mem + slot_bytes);
+  const bool init = !kept || !buf->neutral;
+  if (kept) {
+    keep = buf;
+    buf->neutral = false;  // until this loop's are folded
+  }
+  if (!init) return hipSuccess;
   hipLaunchKernelGGL(k_series_init, dim3(64), dim3(256), 0, s, slots, held);
   return hipGetLastError();
 }
@@ -650,10 +662,12 @@ void SeriesRun::taken(int64_t i, int64_t k, hipStream_t s) {
                      folded + 3 * first);
 }
 
-hipError_t SeriesRun::fetch(double* out, hipStream_t s) const {
-  const hipError_t e =
+hipError_t SeriesRun::fetch(double* out, hipStream_t s) {
+  hipError_t e =
       hipMemcpyAsync(out, folded, sizeof(double) * 3 * nsteps, hipMemcpyDeviceToHost, s);
-  return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && keep) keep->neutral = true;
+  return e;
 }
 
 template void launch_step<double>(const StepIO<double>&, const StepParams&, StepSeries, uint64_t,

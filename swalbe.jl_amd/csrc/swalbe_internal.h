@@ -216,17 +216,28 @@ struct StepSeries {
   }
 };
 
+// Device memory for the series of loops of up to kSeriesKeep steps, kept with
+// the film (264 KB): making and freeing it per call cost a loop of one step of a
+// 64 x 64 film 40 of 90 us.
+constexpr int64_t kSeriesKeep = 64;
+struct SeriesBuf {
+  void* mem = nullptr;   // slots of kSeriesKeep steps, then 3 doubles per step
+  bool neutral = false;  // every slot at its neutral value (the fold leaves them so)
+};
+
 // The series of one loop: the slots of kSeriesChunk steps on the device,
 // folded into one {max, min, count} per step whenever they are used up.
 constexpr int64_t kSeriesChunk = 1024;
 struct SeriesRun {
+  void* own = nullptr;        // memory of this loop alone
+  SeriesBuf* keep = nullptr;  // or the film's
   unsigned long long* slots = nullptr;
   double* folded = nullptr;  // 3 per step
   int64_t nsteps = 0;
   int dh = 0, wet = 0;
   ~SeriesRun();
   bool on() const { return slots != nullptr; }
-  hipError_t start(int64_t n, bool want_dh, bool want_wet, hipStream_t s);
+  hipError_t start(int64_t n, bool want_dh, bool want_wet, SeriesBuf* buf, hipStream_t s);
   // slots of step i (from 0); a launch takes at most room(i) steps from it
   StepSeries at(int64_t i) const {
     return {slots ? slots + (i % kSeriesChunk) * kSeriesSlots * kSeriesWords : nullptr, dh, wet};
@@ -234,7 +245,7 @@ struct SeriesRun {
   int64_t room(int64_t i) const { return slots ? kSeriesChunk - i % kSeriesChunk : INT64_MAX; }
   void taken(int64_t i, int64_t k, hipStream_t s);  // after the launch of steps i .. i + k - 1
   // {max, min, count} of every step on the host
-  hipError_t fetch(double* out, hipStream_t s) const;
+  hipError_t fetch(double* out, hipStream_t s);
 };
 
 template <typename T>
