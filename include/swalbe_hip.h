@@ -445,8 +445,9 @@ typedef struct swalbe1d_step_opts {
     int32_t body;            /* inclination!(α, state) after the force sum */
     int32_t bound;           /* bounce-back walls (BORDER1/2); mass Σ(h - interior h) */
     int32_t materialize;     /* afterwards pressure, h∇p, slip, kbt, F, feq hold the last step's */
-    int32_t variant;         /* 0 = several steps per launch in registers (with `threads` set:
-                                resident when the film fits in LDS, else one launch per step);
+    int32_t variant;         /* 0 = several steps per launch in registers (with `threads` set,
+                                or mass records or snapshots every few steps: resident when the
+                                film fits in LDS; `threads` set and longer: one launch per step);
                                 1 = one launch per step; 2 = resident (error if too big);
                                 every variant gives the same fields */
     uint64_t seed;
@@ -464,7 +465,11 @@ typedef struct swalbe1d_step_opts {
 } swalbe1d_step_opts;
 int swalbe1d_time_loop(swalbe_film1d *st, const swalbe_params *p, int64_t nsteps,
                        const swalbe1d_step_opts *opts);
-/* Same, reporting the device time of the loop (HIP events on the film's stream). */
+/* The kernel that swalbe1d_time_loop takes for this film, loop length and options:
+ * 0 = one launch per step, 1 = several steps per launch, 2 = resident in LDS. */
+int swalbe1d_loop_kernel(swalbe_film1d *st, const swalbe_params *p, int64_t nsteps,
+                         const swalbe1d_step_opts *opts, int32_t *kernel_out);
+/* swalbe1d_time_loop, reporting the device time of the loop (HIP events on the film's stream). */
 int swalbe1d_time_loop_timed(swalbe_film1d *st, const swalbe_params *p, int64_t nsteps,
                              const swalbe1d_step_opts *opts, double *ms_out);
 /* Many 1D films stepped together in one launch, one workgroup per film,

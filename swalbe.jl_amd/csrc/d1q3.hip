@@ -1204,10 +1204,8 @@ int refresh_kappa(swalbe_film1d* s, int n, int m, double hmin) {
 
 int64_t count_every(int64_t t0, int64_t nsteps, int64_t every) {
   if (every <= 0) return 0;
-  int64_t k = 0;
-  for (int64_t it = 1; it <= nsteps; ++it)
-    if ((t0 + it) % every == 0) ++k;
-  return k;
+  auto multiples = [&](int64_t t) { return t / every - (t % every < 0); };  // at most t
+  return multiples(t0 + nsteps) - multiples(t0);
 }
 
 // the per-film description for the fused kernels; the loop's input moments
@@ -1742,6 +1740,37 @@ void launch_wave(const Film1& S, uint64_t step, int npt, int k, swalbe::StepSeri
   else launch_wave_n<T, 1>(S, step, k, ser, st);
 }
 
+// Whether a film that fits in LDS is stepped faster there than by k1_wave, whose
+// launches every mass record and snapshot cuts: the host's work on a cut (a record's
+// step and sum, a snapshot's copy) is longer than the steps between cuts that are few
+// steps apart.  us per step of each kernel, fitted to 2590 measured loops: 64 to 3300
+// nodes, a record, a snapshot or both every 1 to 64 steps or none, both types, τ and
+// noise, 64 and 640 steps; 13 % in the waves' favour, since hosts differ (the same
+// loop's cuts by up to 30 %).  What it picks is on average within 0.5 % of the faster
+// kernel's time and at most 1.30 times it.  Measured, k1_wave / in LDS, 640 FP64
+// steps: L = 64 with a record every 1, 2, 4, 6 steps 8.3 / 2.3, 4.2 / 2.2, 2.2 / 2.1,
+// 1.5 / 2.1, with a snapshot 7.4 / 1.7, 3.2 / 1.4, 1.7 / 1.2, 1.2 / 1.2; L = 1000 with
+// a record every 1, 2 steps 7.8 / 4.7, 4.3 / 4.6, with a snapshot every 1, 3, 5 steps
+// 10.1 / 3.3, 2.4 / 2.3, 1.5 / 2.1; L = 3300 with a snapshot every 1, 2 steps 16.9 /
+// 8.4, 4.8 / 6.4, with noise too 16.9 / 14.7, 4.7 / 12.7.
+bool resident_is_faster(const swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
+                        const swalbe1d_step_opts* o) {
+  if (nsteps < 1) return false;
+  const double n = (double)nsteps, kL = 1e-3 * s->L;
+  const double masses = o->mass_series ? (double)count_every(o->t0, nsteps, p->tdump) / n : 0.0;
+  const double snaps = o->snap_series ? (double)count_every(o->t0, nsteps, o->snap_every) / n : 0.0;
+  if (masses + snaps == 0.0) return false;
+  double wave = 0.18 + 20.0 / n + (6.6 + 0.59 * kL) * masses;
+  wave += (5.5 + 0.1 * (double)s->esz * kL) * snaps;
+  double lds = masses == 0.0 ? 0.89 + 0.61 * kL : s->L <= 512 ? 2.1 : 3.19 + 1.3 * kL;
+  lds += (0.5 + 0.9 * kL) * snaps;
+  if (o->thermal) {
+    wave += 0.64;
+    lds += 0.6 + 1.6 * kL;
+  }
+  return lds < 0.87 * wave;
+}
+
 // The loop in launches of k1_step (any L) or, with `wave`, of k1_wave for
 // every step but the last (and but the steps that a mass record or snapshot
 // falls between); the moments and distributions ping-pong between the two
@@ -1943,7 +1972,35 @@ int loop_resident(swalbe_film1d* const* films, int nfilms, const swalbe_params* 
 
 }  // namespace
 
+namespace {
+
+enum Loop1D { kLoopSteps = 0, kLoopWave = 1, kLoopResident = 2 };
+
+// `threads` asks for one of the two kernels that take it
+Loop1D loop_kernel1(const swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
+                    const swalbe1d_step_opts* o) {
+  if (o->variant == 2) return kLoopResident;
+  if (o->variant != 0) return kLoopSteps;
+  if (fits_resident(s, p) && (o->threads || resident_is_faster(s, p, nsteps, o)))
+    return kLoopResident;
+  return o->threads ? kLoopSteps : kLoopWave;
+}
+
+}  // namespace
+
 extern "C" {
+
+int swalbe1d_loop_kernel(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
+                         const swalbe1d_step_opts* o, int32_t* kernel_out) {
+  if (!s || !p || !kernel_out || nsteps < 0) return bad1("swalbe1d_loop_kernel: bad arguments");
+  swalbe1d_step_opts zero{};
+  if (!o) o = &zero;
+  if (int rc = check_opts(s, p, o)) return rc;
+  if (o->variant == 2 && !fits_resident(s, p))
+    return bad1("swalbe1d_loop_kernel: the film does not fit in LDS (variant 2)");
+  *kernel_out = loop_kernel1(s, p, nsteps, o);
+  return SWALBE_OK;
+}
 
 int swalbe1d_time_loop(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
                        const swalbe1d_step_opts* o) {
@@ -1954,15 +2011,15 @@ int swalbe1d_time_loop(swalbe_film1d* s, const swalbe_params* p, int64_t nsteps,
   (void)hipSetDevice(s->device);
   if (o->variant == 2 && !fits_resident(s, p))
     return bad1("swalbe1d_time_loop: the film does not fit in LDS (variant 2)");
-  // `threads` asks for one of the two kernels that take it
-  const bool resident = o->variant == 2 || (o->variant == 0 && o->threads && fits_resident(s, p));
+  const Loop1D kernel = loop_kernel1(s, p, nsteps, o);
+  const bool resident = kernel == kLoopResident;
   int rc;
   if (resident) {
     rc = loop_resident(&s, 1, p, nsteps, &o, s->stream, nullptr);
   } else {
     if (o->use_theta_field)
       if ((rc = refresh_kappa(s, p->n, p->m, p->hmin))) return rc;
-    rc = loop_per_step(s, p, nsteps, o, o->variant == 0 && !o->threads);
+    rc = loop_per_step(s, p, nsteps, o, kernel == kLoopWave);
   }
   if (rc == SWALBE_OK && o->materialize && nsteps > 0 && !resident) {
     materialize(s, p, o, nsteps);

@@ -219,6 +219,8 @@ def lib():
     _sig(L, "swalbe1d_force_sum", [_V, _I, _I])
     _sig(L, "swalbe1d_reduce", [_V, _I, _D, _I, C.POINTER(_D)])
     _sig(L, "swalbe1d_time_loop", [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts1D)])
+    _sig(L, "swalbe1d_loop_kernel",
+         [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts1D), C.POINTER(_I)])
     _sig(L, "swalbe1d_time_loop_timed",
          [_V, C.POINTER(Params), C.c_int64, C.POINTER(StepOpts1D), C.POINTER(_D)])
     _sig(L, "swalbe1d_ensemble_time_loop",
